@@ -69,40 +69,51 @@ __host__ __device__ inline void moments_acc(const T* f, T& rho, T& v0, T& v1, T&
   if constexpr (S + 1 < Q) moments_acc<Q, T, S + 1>(f, rho, v0, v1, v2);
 }
 
+// Relaxation of the direction pairs (S, opp(S)), S counting up, and the rest
+// direction.  The opposite direction's c . v and c . F are the exact negatives,
+// so the products that are even in them are formed once per pair (D3Q19 FP64 at
+// F = 0: 236 instead of 269 FP64 instructions per collision); every value is
+// rounded as the reference rounds it.
 template <int Q, typename T, int S, bool FORCE>
 __host__ __device__ inline void relax_ref(const T* f, T* out, T rho, T v0, T v1, T v2, T vdotv,
                                           T fdotv, const T* F, double omega) {
 #pragma clang fp contract(off)
   using D = Dir<Q, S>;
+  constexpr int O = Lattice<Q>::opp(S);
   const T w = T(Lattice<Q>::w(S));
-  if constexpr (!FORCE) {
-    // F = 0: every Guo term is an exact +0 (cdotf = fdotv = 0), so dropping
-    // them leaves the reference result unchanged bit for bit.
-    if constexpr (D::cx == 0 && D::cy == 0 && D::cz == 0) {
-      T eq = w * rho * (1.0 - 0.5 * vdotv);
-      out[S] = (1.0 - omega) * f[S] + omega * eq;
-    } else {
-      T cdotv = 3.0 * csum<T, D::cx, D::cy, D::cz>(v0, v1, v2);
-      T eq = w * rho * (1.0 + cdotv + 0.5 * cdotv * cdotv - 0.5 * vdotv);
-      out[S] = (1.0 - omega) * f[S] + omega * eq;
-    }
-  } else if constexpr (D::cx == 0 && D::cy == 0 && D::cz == 0) {
+  if constexpr (D::cx == 0 && D::cy == 0 && D::cz == 0) {
     // rest direction: cdotv = cdotf = 0, (1 + 0) + 0 - x == 1 - x exactly
     T eq = w * rho * (1.0 - 0.5 * vdotv);
-    T fdist = w * (T(0) - fdotv);
-    out[S] = (1.0 - omega) * f[S] + omega * eq + (1.0 - 0.5 * omega) * fdist;
-  } else {
-    T cdotv = 3.0 * csum<T, D::cx, D::cy, D::cz>(v0, v1, v2);
-    T cdotf = 3.0 * csum<T, D::cx, D::cy, D::cz>(F[0], F[1], F[2]);
-    T eq = w * rho * (1.0 + cdotv + 0.5 * cdotv * cdotv - 0.5 * vdotv);
-    T fdist = w * (cdotf - fdotv + cdotv * cdotf);
-    out[S] = (1.0 - omega) * f[S] + omega * eq + (1.0 - 0.5 * omega) * fdist;
+    if constexpr (FORCE) {
+      T fdist = w * (T(0) - fdotv);
+      out[S] = (1.0 - omega) * f[S] + omega * eq + (1.0 - 0.5 * omega) * fdist;
+    } else {
+      // F = 0: every Guo term is an exact +0 (cdotf = fdotv = 0), so dropping
+      // them leaves the reference result unchanged bit for bit.
+      out[S] = (1.0 - omega) * f[S] + omega * eq;
+    }
+  } else if constexpr (S < O) {
+    const T cdotv = 3.0 * csum<T, D::cx, D::cy, D::cz>(v0, v1, v2);
+    const double quad = 0.5 * cdotv * cdotv, half = 0.5 * vdotv;
+    const T eq = w * rho * (1.0 + cdotv + quad - half);
+    const T eqo = w * rho * (1.0 - cdotv + quad - half);
+    if constexpr (FORCE) {
+      const T cdotf = 3.0 * csum<T, D::cx, D::cy, D::cz>(F[0], F[1], F[2]);
+      const T vf = cdotv * cdotf;
+      const T fdist = w * (cdotf - fdotv + vf);
+      const T fdisto = w * (-cdotf - fdotv + vf);
+      out[S] = (1.0 - omega) * f[S] + omega * eq + (1.0 - 0.5 * omega) * fdist;
+      out[O] = (1.0 - omega) * f[O] + omega * eqo + (1.0 - 0.5 * omega) * fdisto;
+    } else {
+      out[S] = (1.0 - omega) * f[S] + omega * eq;
+      out[O] = (1.0 - omega) * f[O] + omega * eqo;
+    }
   }
   if constexpr (S + 1 < Q)
     relax_ref<Q, T, S + 1, FORCE>(f, out, rho, v0, v1, v2, vdotv, fdotv, F, omega);
 }
 
-// In-place or out-of-place: out may alias f (each f[S] is read before out[S] is written).
+// In-place or out-of-place: out may be f itself (each f[S] is read before out[S] is written).
 // FORCE = false requires F = (0, 0, 0) and then equals FORCE = true bit for bit.
 template <int Q, typename T, bool BRINKMAN, bool FORCE = true>
 __host__ __device__ inline void collide_ref(const T* f, T* out, double omega, const T* F,
@@ -147,27 +158,35 @@ __host__ __device__ inline void moments_shift(const float* d, double& drho, doub
   if constexpr (S + 1 < Q) moments_shift<Q, S + 1>(d, drho, m0, m1, m2);
 }
 
+// Relaxation of the direction pairs (S, opp(S)) of the deviations.  The part of
+// the update that is even in c and the odd part are formed once per pair (D3Q19
+// at F = 0: 209 instead of 268 instructions per collision, moments included);
+// every FMA is written out, so that each kernel that collides rounds alike.
+//   even = om (drho + rho (cu^2/2 - uu/2)) + omf (cu cf - fu),  odd = om rho cu + omf cf
+// with uh = uu / 2, r = om rho and omd = om drho - omf fu.
 template <int Q, int S, bool FORCE>
-__host__ __device__ inline void relax_shift(float* d, float drho, float rho, float u0, float u1,
-                                            float u2, float uu, float fu, float F0, float F1,
-                                            float F2, float om, float omf) {
-#pragma clang fp contract(fast)
+__host__ __device__ inline void relax_shift(float* d, float omd, float r, float a0, float a1,
+                                            float a2, float uh, float b0, float b1, float b2,
+                                            float keep, float omf) {
   using D = Dir<Q, S>;
+  constexpr int O = Lattice<Q>::opp(S);
   constexpr float w = (float)Lattice<Q>::w(S);
-  float cu = 0.0f, cf = 0.0f;
-  if constexpr (!(D::cx == 0 && D::cy == 0 && D::cz == 0)) {
-    cu = 3.0f * csum<float, D::cx, D::cy, D::cz>(u0, u1, u2);
-    if constexpr (FORCE) cf = 3.0f * csum<float, D::cx, D::cy, D::cz>(F0, F1, F2);
-  }
-  const float eqdev = drho + rho * (cu + 0.5f * cu * cu - 0.5f * uu);
-  if constexpr (FORCE) {
-    const float fd = cf - fu + cu * cf;
-    d[S] = (1.0f - om) * d[S] + w * (om * eqdev + omf * fd);
-  } else {
-    d[S] = (1.0f - om) * d[S] + w * (om * eqdev);
+  if constexpr (D::cx == 0 && D::cy == 0 && D::cz == 0) {
+    d[S] = __builtin_fmaf(w, __builtin_fmaf(-r, uh, omd), keep * d[S]);
+  } else if constexpr (S < O) {
+    const float cu = csum<float, D::cx, D::cy, D::cz>(a0, a1, a2);
+    float even = __builtin_fmaf(r, __builtin_fmaf(0.5f * cu, cu, -uh), omd);
+    float odd = r * cu;
+    if constexpr (FORCE) {
+      const float cf = omf * csum<float, D::cx, D::cy, D::cz>(b0, b1, b2);
+      even = __builtin_fmaf(cu, cf, even);
+      odd += cf;
+    }
+    d[S] = __builtin_fmaf(w, even + odd, keep * d[S]);
+    d[O] = __builtin_fmaf(w, even - odd, keep * d[O]);
   }
   if constexpr (S + 1 < Q)
-    relax_shift<Q, S + 1, FORCE>(d, drho, rho, u0, u1, u2, uu, fu, F0, F1, F2, om, omf);
+    relax_shift<Q, S + 1, FORCE>(d, omd, r, a0, a1, a2, uh, b0, b1, b2, keep, omf);
 }
 
 // d[Q]: deviations f_s - w_s in FP32, updated in place.  FORCE = false requires F = 0.
@@ -187,13 +206,18 @@ __host__ __device__ inline void collide_shifted(float* d, double omega, const do
     u2 *= (1.0 - gamma);
   }
   const float fu0 = (float)u0, fu1 = (float)u1, fu2 = (float)u2;
-  const float F0 = (float)F[0], F1 = (float)F[1], F2 = (float)F[2];
-  const float uu = 3.0f * (fu0 * fu0 + fu1 * fu1 + fu2 * fu2);
-  const float fu = 3.0f * (F0 * fu0 + F1 * fu1 + F2 * fu2);
-  const float om = (float)omega;
-  const float omf = 1.0f - 0.5f * om;
-  relax_shift<Q, 0, FORCE>(d, (float)drho, (float)rho, fu0, fu1, fu2, uu, fu, F0, F1, F2, om,
-                           omf);
+  const float om = (float)omega, omf = 1.0f - 0.5f * om;
+  const float uh = 1.5f * __builtin_fmaf(fu2, fu2, __builtin_fmaf(fu1, fu1, fu0 * fu0));
+  float omd = om * (float)drho;
+  float F0 = 0.0f, F1 = 0.0f, F2 = 0.0f;  // 3 F
+  if constexpr (FORCE) {
+    F0 = 3.0f * (float)F[0];
+    F1 = 3.0f * (float)F[1];
+    F2 = 3.0f * (float)F[2];
+    omd = __builtin_fmaf(-omf, __builtin_fmaf(F2, fu2, __builtin_fmaf(F1, fu1, F0 * fu0)), omd);
+  }
+  relax_shift<Q, 0, FORCE>(d, omd, om * (float)rho, 3.0f * fu0, 3.0f * fu1, 3.0f * fu2, uh, F0, F1,
+                           F2, 1.0f - om, omf);
 }
 
 }  // namespace lbm

@@ -553,8 +553,29 @@ lbm_status enqueue_aa_pair_by_slabs(lbm_dense* h) {
   return run(K_AA_ODD, S - 1);
 }
 
+// Whether a caller records the handle's stream into a graph of its own.
+bool caller_captures(const lbm_dense* h) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (h->own_capture) return false;
+  if (hipStreamIsCapturing(h->stream, &s) != hipSuccess) (void)hipGetLastError();
+  return s == hipStreamCaptureStatusActive;
+}
+
 lbm_status enqueue_steps(lbm_dense* h, int nsteps) {
-  for (int i = 0; i < nsteps; i++) {
+  int i = 0;
+  if (h->pair.launch) {
+    // A caller's graph of an even run has to end in the array it starts in, as
+    // with one step per launch, so it records an even number of pairs.
+    int pairs = nsteps / 2;
+    if (pairs % 2 && caller_captures(h)) pairs--;
+    for (; i < 2 * pairs; i += 2) {
+      h->pair.launch(h->stream, h->f[h->cur], h->f[1 - h->cur], h->args, h->pair_args);
+      LBM_LAUNCH_CHECK();
+      h->cur = 1 - h->cur;
+      h->t += 2;
+    }
+  }
+  for (; i < nsteps; i++) {
     lbm_status st;
     if (h->pattern == LBM_PATTERN_AA && h->slab_planes > 0 && h->t % 2 == 0 && i + 1 < nsteps) {
       st = enqueue_aa_pair_by_slabs(h);
@@ -612,8 +633,80 @@ lbm_status init_from(lbm_dense* h, int src_kind, const double* rho_d, const doub
   return LBM_OK;
 }
 
+// Number of planes per chunk of the two-step kernel: the launch takes as many
+// rounds as the resident workgroups need for all work items, and a round as long
+// as a chunk's planes and its two halo planes (and about half a plane to start).
+// With this rule a 256^3 D3Q19 FP64 box runs 256-plane chunks, 493 us per step
+// (64 planes: 545); 100^3 runs 12-plane chunks, 39.8 us (64 planes: 152).
+PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
+  PairArgs p{};
+  p.ntx = (nx + k.w - 1) / k.w;
+  p.nty = (ny + k.ty - 1) / k.ty;
+  double best = 0.0;
+  for (int lz = 1; lz <= nz; lz++) {
+    const int64_t items = (int64_t)p.ntx * p.nty * ((nz + lz - 1) / lz);
+    const double cost = (double)((items + slots - 1) / slots) * (lz + 2.5);
+    if (lz == 1 || cost < best) {
+      best = cost;
+      p.lz = lz;
+    }
+  }
+  p.nch = (nz + p.lz - 1) / p.lz;
+  p.per_xcd = (int)(((int64_t)p.ntx * p.nty * p.nch + 7) / 8);
+  return p;
+}
+
+// Two steps per launch (lbm_dense_pair.hpp) on unmasked periodic SOA boxes in
+// FP64 and FP32 deviations, without per-cell fields or a pressure drop.  Default
+// from 20,000 cells on; below, the march along z is a longer chain than two
+// launches (us per step, one step / two steps per launch, D3Q19 FP64: 16^3 3.9 /
+// 4.6, 128 x 16 x 8 3.8 / 5.4, 24^3 5.0 / 4.8, 28^3 6.3 / 5.0, 12 x 12 x 200
+// 11.6 / 7.2; every larger size measured gained).  LBM_DENSE_PAIR=0|1 overrides;
+// a variable that tunes the one-step kernels asks for them.  Sets h->pair and
+// h->pair_args, and the cache policy: stores stream past the caches when both
+// arrays exceed 320 MiB (100^3 FP64, 290 MiB: 44.0 us cached / 44.7 streaming;
+// 112^3, 408 MiB: 54.4 / 52.9; 120^3 FP32, 250 MiB: 34.4 / 39.8).
+void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links) {
+  const char* e = std::getenv("LBM_DENSE_PAIR");
+  bool on = h->ncell >= 20000;
+  for (const char* v : {"LBM_DENSE_IROWS", "LBM_DENSE_ODD_SEG", "LBM_DENSE_SLAB_PLANES",
+                        "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS"})
+    on = on && !std::getenv(v);
+  if (e) on = e[0] != '0';
+  const size_t plane_bytes = (size_t)h->nx * h->ny * h->esize;
+  if (!on || need_links || h->layout != LBM_LAYOUT_SOA || cfg->tau || cfg->gamma ||
+      cfg->density_jump_x != 0.0 || plane_bytes > UINT32_MAX)
+    return;
+  const bool force = cfg->force[0] != 0.0 || cfg->force[1] != 0.0 || cfg->force[2] != 0.0;
+  bool nt = h->nt;
+  if (!std::getenv("LBM_DENSE_NT"))
+    nt = 2 * (size_t)h->ncell * h->q * h->esize > ((size_t)320 << 20);
+  const auto pick = h->q == 19 ? pick_pair19 : pick_pair27;
+  auto slots = [](const PairKernel& k) {
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, k.threads, k.lds) != hipSuccess)
+      return 0;
+    return cus * per_cu;
+  };
+  const bool narrow = h->nx <= 32;
+  // Small tiles where single planes of the large ones do not fill the GPU (32^3
+  // D3Q19 FP64: 5.2 us per step against 6.7; 48^3, where they do: 9.6 / 8.7).
+  for (const bool small : {false, true}) {
+    const PairKernel k = pick(h->storage, force, nt, narrow, small);
+    const int s = k.launch ? slots(k) : 0;
+    if (s <= 0) return;
+    const PairArgs p = plan_pair(k, h->nx, h->ny, h->nz, s);
+    if ((int64_t)p.ntx * p.nty * p.nch >= ((int64_t)1 << 28)) return;
+    h->pair = k;
+    h->pair_args = p;
+    if ((int64_t)p.ntx * p.nty * h->nz > s) return;
+  }
+}
+
 lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_by_gather,
-                        bool irows_ok) {
+                        bool irows_ok, bool pair_ok) {
   LBM_REQUIRE(cfg && out, LBM_ERR_ARG, "lbm_dense_create: null pointer");
   *out = nullptr;
   LBM_REQUIRE(cfg->nx > 0 && cfg->ny > 0 && cfg->nz > 0, LBM_ERR_ARG,
@@ -658,6 +751,22 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   const bool need_links =
       cfg->solid != nullptr || !h->periodic[0] || !h->periodic[1] || !h->periodic[2];
   if (need_links) h->odd_seg_w = 0;  // the segmented odd step covers unmasked periodic boxes
+  // Two steps per launch work out of place, in the AB pull convention.  For an AA
+  // box they take a second population array, so only while both fit easily: a
+  // quarter of the GPU's memory, and half of what is free (512^3 D3Q19 FP64:
+  // 41 of 288 GB).  Larger boxes, and a GPU that is nearly full, step in place.
+  if (pair_ok) choose_pair(h, cfg, need_links);
+  const bool aa_as_pairs = h->pair.launch && h->pattern == LBM_PATTERN_AA;
+  if (aa_as_pairs) {
+    size_t room = 0, total = 0;
+    const size_t both = 2 * (size_t)h->ncell * h->q * h->esize;
+    if (hipMemGetInfo(&room, &total) != hipSuccess || both > total / 4 || both > room / 2)
+      h->pair = {};
+  }
+  if (h->pair.launch) {
+    h->pattern = LBM_PATTERN_AB;
+    h->pull = 1;
+  }
   // Interleaved rows (lbm_dense_kernels.hpp) for AA on unmasked periodic SOA
   // boxes whose rows are whole 64-element blocks: the odd step then makes only
   // whole aligned block accesses, like the even step.  Per-cell fields are
@@ -717,7 +826,12 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   const size_t fbytes = (size_t)h->ncell * h->q * h->esize;
   const int narrays = h->pattern == LBM_PATTERN_AA ? 1 : 2;
   for (int i = 0; i < narrays; i++)
-    if ((st = dmalloc(h, &h->f[i], fbytes, "populations"))) return fail(st);
+    if ((st = dmalloc(h, &h->f[i], fbytes, "populations"))) {
+      (void)fail(st);
+      return aa_as_pairs && narrays == 2
+                 ? dense_create(cfg, out, push_by_gather, irows_ok, false)  // in place after all
+                 : st;
+    }
   if ((st = dmalloc(h, (void**)&h->partial, sizeof(double) * (h->npartial + 1), "reduction")))
     return fail(st);
   if (need_links) {
@@ -824,7 +938,8 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   }
   // rest state, as PropagationAA/AB::initialize (src/propagation/PropagationAA.cpp:60-123)
   if ((st = init_from(h, 0, nullptr, nullptr, 0.0, 0.0, 0))) return fail(st);
-  if (h->pattern == LBM_PATTERN_AB &&
+  // (the two-step kernels store every cell of the second array before it is read)
+  if (h->pattern == LBM_PATTERN_AB && !h->pair.launch &&
       hipMemcpyAsync(h->f[1], h->f[0], fbytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) {
     set_error("lbm_dense_create: initial copy failed");
     return fail(LBM_ERR_HIP);
@@ -842,7 +957,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
 extern "C" {
 
 lbm_status lbm_dense_create(const lbm_dense_config* cfg, lbm_dense** out) {
-  return dense_create(cfg, out, true, true);
+  return dense_create(cfg, out, true, true, true);
 }
 
 lbm_status lbm_dense_destroy(lbm_dense* h) {
@@ -966,28 +1081,31 @@ lbm_status lbm_dense_set_stream(lbm_dense* h, void* stream) {
 }
 
 // A captured run of an even number of steps.  After an even number of steps
-// the AA array is back in the convention it started in and the AB pair has
-// swapped twice, so one replay continues the run from any state whose phase
-// (t mod 2 for AA, the current array for AB) equals the phase at capture.
-// The kernels take the handle's device pointers, which stay fixed for the
-// handle's lifetime; capture records kernel launches only.
+// every convention holds its states as it did before, so a replay continues the
+// run from any state an even number of steps from the one at capture.  The
+// out-of-place kernels read one array and write the other: one step per launch
+// brings an even run back to the array it started in, but two steps per launch
+// may not, and the handle may have changed arrays since the capture, so a
+// handle with two-step launches captures the run once from each array and
+// replays the one that starts in the current array.  The kernels take the
+// handle's device pointers, which stay fixed for the handle's lifetime; capture
+// records kernel launches only.
 struct lbm_dense_graph {
   lbm_dense* h = nullptr;
   int32_t nsteps = 0;
-  int phase = 0;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  bool counted = false;  // included in h->live_graphs
+  int phase = 0;                             // parity of the step at capture
+  hipGraph_t graph[2] = {nullptr, nullptr};  // by the array the run starts in
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  int end[2] = {0, 0};                       // the array it ends in
+  bool counted = false;                      // included in h->live_graphs
 };
-
-static int dense_phase(const lbm_dense* h) {
-  return h->pattern == LBM_PATTERN_AA ? (int)(h->t % 2) : h->cur;
-}
 
 lbm_status lbm_dense_graph_destroy(lbm_dense_graph* g) {
   if (!g) return LBM_OK;
-  if (g->exec) (void)hipGraphExecDestroy(g->exec);
-  if (g->graph) (void)hipGraphDestroy(g->graph);
+  for (int c = 0; c < 2; c++) {
+    if (g->exec[c]) (void)hipGraphExecDestroy(g->exec[c]);
+    if (g->graph[c]) (void)hipGraphDestroy(g->graph[c]);
+  }
   if (g->counted) g->h->live_graphs--;
   delete g;
   return LBM_OK;
@@ -1001,7 +1119,7 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
   auto* g = new lbm_dense_graph;
   g->h = h;
   g->nsteps = nsteps;
-  g->phase = dense_phase(h);
+  g->phase = (int)(h->t % 2);
   // capture on a stream of its own: the caller's stream may be the null
   // stream, which cannot be captured, and nothing captured runs now
   hipStream_t cap = nullptr;
@@ -1015,20 +1133,26 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
   const int64_t t0 = h->t;
   const int cur0 = h->cur;
   h->stream = cap;
+  h->own_capture = true;
   lbm_status st = LBM_OK;
-  e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
+  for (int c = 0; c < 2 && st == LBM_OK && e == hipSuccess; c++) {
+    if (!h->pair.launch && c != cur0) continue;
+    h->t = t0;
+    h->cur = c;
+    e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) break;
     st = enqueue_steps(h, nsteps);
-    hipGraph_t graph = nullptr;
-    const hipError_t e2 = hipStreamEndCapture(cap, &graph);
-    g->graph = graph;
+    const hipError_t e2 = hipStreamEndCapture(cap, &g->graph[c]);
     if (st == LBM_OK && e2 != hipSuccess) e = e2;
+    if (st == LBM_OK && e == hipSuccess)
+      e = hipGraphInstantiate(&g->exec[c], g->graph[c], nullptr, nullptr, 0);
+    g->end[c] = h->cur;
   }
   h->stream = user;
+  h->own_capture = false;
   h->t = t0;
   h->cur = cur0;
   (void)hipStreamDestroy(cap);
-  if (st == LBM_OK && e == hipSuccess) e = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
   if (st != LBM_OK || e != hipSuccess) {
     if (st == LBM_OK) set_error("lbm_dense_graph_create: %s", hipGetErrorString(e));
     lbm_dense_graph_destroy(g);
@@ -1043,11 +1167,12 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
 lbm_status lbm_dense_graph_launch(lbm_dense_graph* g, int32_t nlaunch) {
   LBM_REQUIRE(g && nlaunch >= 0, LBM_ERR_ARG, "lbm_dense_graph_launch: bad arguments");
   lbm_dense* h = g->h;
-  LBM_REQUIRE(dense_phase(h) == g->phase, LBM_ERR_ARG,
+  LBM_REQUIRE((int)(h->t % 2) == g->phase && g->exec[h->cur], LBM_ERR_ARG,
               "lbm_dense_graph_launch: the handle is an odd number of steps away from the "
               "state the graph was captured in");
   for (int32_t i = 0; i < nlaunch; i++) {
-    LBM_HIP_CHECK(hipGraphLaunch(g->exec, h->stream));
+    LBM_HIP_CHECK(hipGraphLaunch(g->exec[h->cur], h->stream));
+    h->cur = g->end[h->cur];
     h->t += g->nsteps;
   }
   return LBM_OK;

@@ -1,7 +1,7 @@
 // lbm_dense_internal.hpp -- the dense engine handle and the host helpers that
 // the adjoint module (lbm_adjoint.hip) shares with lbm_dense.hip.
 #pragma once
-#include "lbm_dense_kernels.hpp"
+#include "lbm_dense_pair.hpp"
 
 struct lbm_dense {
   int nx = 0, ny = 0, nz = 0, q = 19, pattern = 1, pull = 0, layout = 0, storage = 0;
@@ -21,6 +21,9 @@ struct lbm_dense {
   int xk = 0;                // interleaved rows: nx / 64 (0: plain rows)
   int odd_ir_bx = 256;       // launch shape of the odd step on interleaved rows
   size_t odd_ir_lds = 0;
+  lbm::PairKernel pair{};  // two time steps per launch (k_dense_pair); launch == nullptr: off
+  lbm::PairArgs pair_args{};
+  bool own_capture = false;  // lbm_dense_graph_create is recording
   int64_t ncell = 0, nfluid = 0, t = 0;
   size_t esize = 8;
   void* f[2] = {nullptr, nullptr};
@@ -53,8 +56,8 @@ lbm_status dmalloc(lbm_dense* h, void** p, size_t bytes, const char* what);
 // lbm_dense_create; push_by_gather = false keeps AB push handles on the
 // scatter kernel and the push storage convention, irows_ok = false keeps plain
 // rows (the adjoint drives the push kernel on the handle's arrays itself and
-// indexes them by cell)
+// indexes them by cell), pair_ok = false keeps one step per launch
 lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_by_gather,
-                        bool irows_ok);
+                        bool irows_ok, bool pair_ok);
 
 }  // namespace lbm

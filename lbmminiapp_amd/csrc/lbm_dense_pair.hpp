@@ -1,0 +1,294 @@
+// lbm_dense_pair.hpp -- two time steps in one pass over memory.
+//
+// A time step reads and writes every population once and does about one
+// operation per byte, so on its own it runs at the copy rate of the memory
+// (D3Q19 FP64 512^3: 40.8 GB in 7.1 ms, 5.8 TB/s, 0.88 of a copy) and only
+// moving less can make it faster.  k_dense_pair advances two steps per read and
+// write of the state: the intermediate populations live in registers and LDS.
+//
+// Storage is the AB pull convention (post-collision values, a step gathers slot
+// s at x - c_s), out of place: reads are the x-shifted ones and go through the
+// caches, where neighbouring workgroups share them; writes are whole aligned
+// row segments.  A handle that the caller created as AA or AB push runs it too
+// (dense_create): every convention holds the same states, bit for bit.
+//
+// A workgroup owns a tile of W x TY cells in (x, y) and marches along z through
+// a chunk of lz planes.  At plane p it
+//   1. collides the tile and a ring of one cell around it (first step) from
+//      registers loaded one plane ahead, and puts the results that change lane
+//      (c_x or c_y != 0) into LDS;
+//   2. starts the loads of plane p + 1;
+//   3. gathers from LDS what the tile's cells receive from plane p: the c_z < 0
+//      part completes plane p - 1, whose second step is collided and stored; the
+//      c_z = 0 and c_z > 0 parts wait in registers for planes p and p + 1.
+// One plane of the Q - 3 exchanged directions is all the LDS holds, so the tile
+// can be large: the ring costs (W + 2)(TY + 2) / (W TY), 1.29 for 64 x 8, in
+// the first step's arithmetic; in memory traffic the caches absorb most of it
+// (measured, 512^3 D3Q19 FP64: 23.0 GB read where the state is 20.4, 20.4
+// written).
+//
+// Waves: W TY / 64 of tile rows, 2 W / 64 of the rows above and below, one of
+// the two columns beside the tile.  Only the tile's waves do the second step.
+// The two roles have loops of their own, and a lane without a cell repeats its
+// neighbour's: with no branch around loads and stores the compiler can count
+// them, and the wait for plane p + 1's loads leaves the stores of plane p - 1 in
+// flight (one loop with the second step in a branch: 4.6 ms per step at 512^3
+// FP64, where two loops take 4.1).
+//
+// Work items go to the XCDs in contiguous runs (x fastest, then y, then chunks),
+// so that the tiles whose rings overlap share an L2.
+//
+// Measured, ms per step, one-step kernels -> pairs (tile as choose_pair takes it):
+//   D3Q19 FP64 512^3 7.15 -> 4.10   256^3 0.912 -> 0.493   128^3 0.110 -> 0.067
+//   D3Q19 FP32 512^3 3.42 -> 2.38   256^3 0.409 -> 0.266
+//   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 384^3 2.40 -> 1.51
+#pragma once
+#include "lbm_dense_kernels.hpp"
+
+namespace lbm {
+
+// Launch geometry of k_dense_pair.
+struct PairArgs {
+  int ntx, nty, nch;  // tiles along x and y, chunks along z
+  int lz;             // planes per chunk
+  int per_xcd;        // work items per XCD (the grid is 8 times as large)
+};
+
+// LDS slot of direction s, or -1 where the receiving cell is in the same lane.
+template <int Q>
+__host__ __device__ constexpr int pair_slot(int s) {
+  if (Lattice<Q>::c(s, 0) == 0 && Lattice<Q>::c(s, 1) == 0) return -1;
+  int k = 0;
+  for (int r = 0; r < s; r++) k += Lattice<Q>::c(r, 0) != 0 || Lattice<Q>::c(r, 1) != 0;
+  return k;
+}
+
+template <int W, int TY>
+constexpr int pair_threads() {
+  return W * TY + 2 * W + 64;
+}
+
+template <int Q, int STORE, int W, int TY>
+constexpr size_t pair_lds_bytes() {
+  return (size_t)(Q - 3) * (W + 2) * (TY + 2) * sizeof(typename Storage<STORE>::C);
+}
+
+// A wave-uniform address kept in scalar registers, so that an access is one
+// instruction with a scalar base and the lane's 32-bit byte offset.
+__device__ __forceinline__ global_ptr<char> scalar_base(const void* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (global_ptr<char>)(((uint64_t)hi << 32) | lo);
+}
+// The lane's offset, opaque next to its use: extended to 64 bits outside the
+// loop it would make every access a 64-bit sum per lane.
+__device__ __forceinline__ uint32_t lane_offset(uint32_t v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
+template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+__global__ void __launch_bounds__((pair_threads<W, TY>()))
+    k_dense_pair(const typename Storage<STORE>::T* __restrict__ f0,
+                 typename Storage<STORE>::T* __restrict__ f1, DenseArgs a, PairArgs pa) {
+  using T = typename Storage<STORE>::T;
+  using C = typename Storage<STORE>::C;
+  static_assert(sizeof(T) == sizeof(C), "the first step's results are kept unrounded");
+  constexpr int EX = W + 2, EY = TY + 2, PL = EX * EY;
+  extern __shared__ unsigned char lbm_smem[];
+  C* lds = reinterpret_cast<C*>(lbm_smem);  // [Q - 3][EY][EX]
+
+  int t = (blockIdx.x & 7) * pa.per_xcd + (blockIdx.x >> 3);
+  if (t >= pa.ntx * pa.nty * pa.nch) return;
+  const int x0 = t % pa.ntx * W;
+  t /= pa.ntx;
+  const int y0 = t % pa.nty * TY;
+  const int zc = t / pa.nty * pa.lz, ze = zc + pa.lz < a.nz ? zc + pa.lz : a.nz;
+  const int xe = x0 + W < a.nx ? x0 + W : a.nx, ye = y0 + TY < a.ny ? y0 + TY : a.ny;
+
+  // The lane's cell (X, Y), which may lie one outside the box (the wrapped
+  // neighbour); lanes past the end of the tile or of their role repeat a cell.
+  constexpr int RW = 64 / W;   // rows per wave
+  constexpr int NI = TY / RW;  // waves of tile rows
+  static_assert(W <= 64 && 64 % W == 0 && TY % RW == 0 && 2 * EY <= 64, "tile shape");
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  int X = x0 + lane % W < xe ? x0 + lane % W : xe - 1, Y;
+  bool inner = false;  // the wave does the second step
+  if (w < NI) {
+    inner = y0 + w * RW < ye;
+    Y = y0 + w * RW + lane / W;
+    Y = inner ? (Y < ye ? Y : ye - 1) : ye;
+  } else if (w < NI + 2 * W / 64) {
+    Y = (w - NI) * RW + lane / W == 0 ? y0 - 1 : ye;
+  } else {
+    const int i = lane < 2 * EY ? lane : 2 * EY - 1;
+    X = i < EY ? x0 - 1 : xe;
+    Y = y0 - 1 + i % EY;
+    Y = Y < ye ? Y : ye;
+  }
+  const int lo = (Y - y0 + 1) * EX + X - x0 + 1;  // the cell's position in an LDS slot
+  const int x = wrap1(X, a.nx), y = wrap1(Y, a.ny);
+  // byte offsets, within a plane, of the cells at (x - cx, y - cy)
+  uint32_t off[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      off[i][j] = ((uint32_t)wrap1(y - (j - 1), a.ny) * (uint32_t)a.nx +
+                   (uint32_t)wrap1(x - (i - 1), a.nx)) * (uint32_t)sizeof(T);
+  const int64_t n = a.ncell, plane = (int64_t)a.nx * a.ny;
+  const double F[3] = {a.F0, a.F1, a.F2};
+
+  auto collide = [&](C* d) {
+    collide_cell<Q, STORE, FORCE, false>(d, a.omega, F, nullptr, 0);
+  };
+  // gathers the populations of plane p (past the chunk: of its last halo plane again)
+  auto load_plane = [&](int p, C(&f)[Q]) {
+    const int z = wrap1(p < ze ? p : ze, a.nz);
+    const int zz[3] = {wrap1(z + 1, a.nz), z, wrap1(z - 1, a.nz)};  // source of cz = -1, 0, 1
+#pragma unroll
+    for (int s = 0; s < Q; s++) {
+      const auto base = scalar_base(f0 + (n * s + plane * zz[Lattice<Q>::c(s, 2) + 1]));
+      f[s] = *(global_ptr<const T>)(
+          base + lane_offset(off[Lattice<Q>::c(s, 0) + 1][Lattice<Q>::c(s, 1) + 1]));
+    }
+  };
+  C own[3];  // the first step's results that stay in the lane, by cz + 1
+  auto first_step = [&](C(&f)[Q]) {
+    collide(f);
+#pragma unroll
+    for (int s = 0; s < Q; s++) {
+      const int k = pair_slot<Q>(s);
+      if (k < 0) own[Lattice<Q>::c(s, 2) + 1] = f[s];
+      else lds[k * PL + lo] = f[s];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  C f[Q];
+  load_plane(zc - 1, f);
+  if (!inner) {
+    for (int p = zc - 1; p <= ze; p++) {
+      first_step(f);
+      load_plane(p + 1, f);
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();  // LDS holds plane p
+      __syncthreads();  // LDS has been read
+    }
+    return;
+  }
+
+  // Populations of the second step: h of cz = 0 and cz = 1 for plane p - 1, and
+  // of cz = 1 for plane p (next), by direction.
+  C h[Q] = {}, next[Q] = {};
+  // what the cell receives in direction s from the plane in LDS
+  auto receive = [&](int s) -> C {
+    const int k = pair_slot<Q>(s);
+    return k < 0 ? own[Lattice<Q>::c(s, 2) + 1]
+                 : lds[k * PL + lo - Lattice<Q>::c(s, 1) * EX - Lattice<Q>::c(s, 0)];
+  };
+  auto second_step = [&](int z) {
+    C d[Q];
+#pragma unroll
+    for (int s = 0; s < Q; s++) d[s] = Lattice<Q>::c(s, 2) < 0 ? receive(s) : h[s];
+    collide(d);
+#pragma unroll
+    for (int s = 0; s < Q; s++) {
+      const auto q = (global_ptr<T>)(scalar_base(f1 + (n * s + plane * z)) + lane_offset(off[1][1]));
+      if constexpr (NT) __builtin_nontemporal_store(d[s], q);
+      else *q = d[s];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto plane_step = [&](int p, auto second) {
+    first_step(f);
+    load_plane(p + 1, f);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();  // LDS holds plane p
+    if constexpr (decltype(second)::value) second_step(p - 1);
+#pragma unroll
+    for (int s = 0; s < Q; s++) {
+      const int cz = Lattice<Q>::c(s, 2);
+      if (cz == 0) {
+        h[s] = receive(s);
+      } else if (cz > 0) {
+        h[s] = next[s];
+        next[s] = receive(s);
+      }
+      // In registers before the barrier that lets the LDS be overwritten: the
+      // compiler has moved such a read, used only later, below the barrier.
+      if (cz == 0) asm volatile("" : "+v"(h[s]));
+      if (cz > 0) asm volatile("" : "+v"(h[s]), "+v"(next[s]));
+    }
+    __syncthreads();  // LDS has been read
+  };
+  plane_step(zc - 1, std::false_type{});
+  plane_step(zc, std::false_type{});
+  for (int p = zc + 1; p <= ze; p++) plane_step(p, std::true_type{});
+}
+
+// A compiled tile shape: its launch, and what a launch plan needs to know of it.
+struct PairKernel {
+  void (*launch)(hipStream_t stream, const void* f0, void* f1, const DenseArgs& a,
+                 const PairArgs& pa);
+  const void* fn;
+  int w, ty, threads;
+  size_t lds;
+};
+
+template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+void launch_pair(hipStream_t stream, const void* f0, void* f1, const DenseArgs& a,
+                 const PairArgs& pa) {
+  using T = typename Storage<STORE>::T;
+  hipLaunchKernelGGL((k_dense_pair<Q, STORE, FORCE, NT, W, TY>), dim3(8 * pa.per_xcd),
+                     dim3(pair_threads<W, TY>()), (pair_lds_bytes<Q, STORE, W, TY>()), stream,
+                     (const T*)f0, (T*)f1, a, pa);
+}
+
+template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+PairKernel pair_kernel() {
+  return {launch_pair<Q, STORE, FORCE, NT, W, TY>,
+          (const void*)k_dense_pair<Q, STORE, FORCE, NT, W, TY>, W, TY, pair_threads<W, TY>(),
+          pair_lds_bytes<Q, STORE, W, TY>()};
+}
+
+template <int Q, int STORE, int W, int TY>
+PairKernel pick_pair_flags(bool force, bool nt) {
+  if (nt) return force ? pair_kernel<Q, STORE, true, true, W, TY>()
+                       : pair_kernel<Q, STORE, false, true, W, TY>();
+  return force ? pair_kernel<Q, STORE, true, false, W, TY>()
+               : pair_kernel<Q, STORE, false, false, W, TY>();
+}
+
+// Tile shapes: W = 64 cells of a row, or 32 for rows of up to 32 (a 24 x 200 x
+// 100 box, D3Q19 FP64: 18.4 us per step with 32 x 16 tiles, 24.1 with 64 x 8).
+// Large tiles have the smaller ring (512^3 D3Q19 FP64, 64 x 8: 4.10 ms per step,
+// 64 x 4: 5.03); the smaller ones give small boxes twice the workgroups.
+// D3Q27 FP64 spills registers in the 11-wave tiles and takes 64 x 4 and 32 x 8
+// always (384^3: 3.09 ms against 3.60).
+template <int Q, int STORE>
+PairKernel pick_pair_tile(bool force, bool nt, bool narrow, bool small) {
+  if constexpr (!(Q == 27 && STORE == LBM_STORE_F64)) {
+    if (!small) return narrow ? pick_pair_flags<Q, STORE, 32, 16>(force, nt)
+                              : pick_pair_flags<Q, STORE, 64, 8>(force, nt);
+  }
+  return narrow ? pick_pair_flags<Q, STORE, 32, 8>(force, nt)
+                : pick_pair_flags<Q, STORE, 64, 4>(force, nt);
+}
+
+template <int Q>
+PairKernel pick_pair_q(int storage, bool force, bool nt, bool narrow, bool small) {
+  switch (storage) {
+    case LBM_STORE_F64: return pick_pair_tile<Q, LBM_STORE_F64>(force, nt, narrow, small);
+    case LBM_STORE_F32S: return pick_pair_tile<Q, LBM_STORE_F32S>(force, nt, narrow, small);
+  }
+  return {};
+}
+
+// Defined in lbm_dense_pair19.hip and lbm_dense_pair27.hip; launch is nullptr
+// where there is no two-step kernel.  narrow: W = 32; small: half the rows.
+PairKernel pick_pair19(int storage, bool force, bool nt, bool narrow, bool small);
+PairKernel pick_pair27(int storage, bool force, bool nt, bool narrow, bool small);
+
+}  // namespace lbm
