@@ -60,13 +60,128 @@ __device__ __forceinline__ int64_t node_block(uint32_t group) {
   return (int64_t)(r / group) * 8 * group + (int64_t)k * group + r % group;
 }
 
+// Node of this work-item.  Node blocks start at multiples of 64, wherever the
+// range starts, so that a wavefront covers one group of kGroup nodes of the
+// compressed adjacency; work-items before the range and past its end idle.
+__device__ __forceinline__ int64_t node_of(int64_t start, uint32_t group) {
+  return (start & ~(int64_t)63) + node_block(group) * blockDim.x + threadIdx.x;
+}
+
+// ---------------------------------------------------------------- adjacency
+// The caller's adjacency costs 4 Q bytes per node and step, 76 of 380 in D3Q19
+// FP64.  In the fluid order of a real geometry the 64 nodes of a group reach
+// their neighbours at a few distances only: within a row of the list the
+// distance adj - own slot is the same, and every bounce-back has one.  So each
+// group holds a table of up to kDeltas distances per direction, and each node a
+// 3-bit code per direction (10 codes a word): 8 + 9.5 bytes per node for D3Q19,
+// built at create on the GPU (k_sparse_compress).  A group with more distances in
+// some direction (about 1 in 1000 at the reference's simulationSize 2, most at
+// 0.5, whose rows are 10 nodes) keeps reading the caller's table.
+// simulationSize 8, D3Q19, us per step, caller's table -> compressed: FP64 AA 573
+// -> 521, push 771 -> 569, pull 653 -> 559; FP32 322 -> 282, 504 -> 336, 387 -> 305.
+// (The push loads its populations before it decodes: 658 us the other way round.)
+constexpr int kGroup = 64;
+constexpr int kDeltas = 8;
+template <int Q>
+__host__ __device__ constexpr int code_words() {
+  return (Q + 9) / 10;
+}
+
+struct AdjTables {
+  const int32_t* adj;    // the caller's adjacency
+  const uint32_t* code;  // [code_words][groups * kGroup]
+  const int32_t* table;  // [groups][Q][kDeltas]
+  const uint32_t* raw;   // [groups]: nonzero where the group is not compressed
+  int64_t groups;
+};
+
+// One wavefront per group.
+template <int Q, int LAYOUT>
+__global__ void __launch_bounds__(kGroup)
+    k_sparse_compress(const int32_t* __restrict__ adj, uint32_t* __restrict__ code,
+                      int32_t* __restrict__ table, uint32_t* __restrict__ raw, int64_t n) {
+  const int64_t g = blockIdx.x;
+  const int lane = threadIdx.x;
+  const int64_t i = g * kGroup + lane;
+  uint32_t words[code_words<Q>()] = {};
+  bool fits = true;
+#pragma unroll
+  for (int s = 0; s < Q; s++) {
+    const int64_t own = pidx<Q, LAYOUT>(n, s, i);
+    const int32_t delta = i < n ? (int32_t)(adj[own] - own) : 0;
+    uint64_t left = __ballot(i < n);
+    uint32_t mine = 0;
+    int32_t entry = 0;
+    for (int k = 0; k < kDeltas && left; k++) {
+      const int32_t d = __builtin_amdgcn_readlane(delta, __builtin_ctzll(left));
+      const uint64_t same = __ballot(delta == d) & left;
+      if ((same >> lane) & 1u) mine = k;
+      if (lane == k) entry = d;
+      left &= ~same;
+    }
+    fits = fits && !left;
+    words[s / 10] |= mine << (3 * (s % 10));
+    if (lane < kDeltas) table[(g * Q + s) * kDeltas + lane] = entry;
+  }
+  for (int w = 0; w < code_words<Q>(); w++) code[(int64_t)w * gridDim.x * kGroup + i] = words[w];
+  if (lane == 0) raw[g] = !fits;
+}
+
+// The adjacency of this work-item's node.  load() and index() take the whole
+// wavefront (a node past the range holds its group's codes too); only index()
+// of a node that exists means something.
+template <int Q, int LAYOUT, bool NT>
+struct AdjReader {
+  static constexpr int kRegs = (Q * kDeltas + 63) / 64;
+  bool raw;
+  uint32_t code[code_words<Q>()];
+  int32_t table[kRegs];  // lane l, register r: entry 64 r + l of the group's table
+
+  __device__ __forceinline__ void load(const AdjTables& t, int64_t i) {
+    const int64_t g = __builtin_amdgcn_readfirstlane((uint32_t)(i / kGroup));
+    raw = t.raw[g] != 0;
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int w = 0; w < code_words<Q>(); w++) code[w] = ldn<NT>(t.code + (w * t.groups * kGroup + i));
+#pragma unroll
+    for (int r = 0; r < kRegs; r++) {
+      const int e = 64 * r + lane;
+      table[r] = ldn<NT>(t.table + (g * Q * kDeltas + (e < Q * kDeltas ? e : Q * kDeltas - 1)));
+    }
+  }
+  __device__ __forceinline__ int32_t index(int s, int64_t n, int64_t i) const {
+    const int c = (code[s / 10] >> (3 * (s % 10))) & (kDeltas - 1);
+    const int d = __builtin_amdgcn_ds_bpermute(4 * ((s * kDeltas) % 64 + c), table[s * kDeltas / 64]);
+    return (int32_t)(pidx<Q, LAYOUT>(n, s, i)) + d;
+  }
+};
+
+// All Q neighbour slots of a node, compressed (COMP; the whole wavefront takes
+// part) or from the caller's table.
+template <int Q, int LAYOUT, bool NT, bool COMP>
+__device__ __forceinline__ void neighbour_slots(const AdjTables& t, int64_t n, int64_t i, bool active,
+                                                int32_t* loc) {
+  if constexpr (COMP) {
+    AdjReader<Q, LAYOUT, NT> r;
+    r.load(t, i);
+    if (!r.raw) {
+#pragma unroll
+      for (int s = 0; s < Q; s++) loc[s] = r.index(s, n, i);
+      return;
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < Q; s++)
+    loc[s] = COMP && !active ? 0 : ldn<NT>(t.adj + pidx<Q, LAYOUT>(n, s, i));
+}
+
 // AA even: src/kernels/KernelAA_SOA_Base.cpp:173-254 (AOS: KernelAA_AOS_Base.cpp:174-254)
 template <int Q, typename T, int LAYOUT, bool NT>
 __global__ void __launch_bounds__(256)
     k_sparse_aa_even(T* __restrict__ f, int64_t n, int64_t start, int64_t count, double omega,
                      T F0, T F1, T F2, uint32_t group) {
-  const int64_t i = start + node_block(group) * blockDim.x + threadIdx.x;
-  if (i >= start + count) return;
+  const int64_t i = node_of(start, group);
+  if (i < start || i >= start + count) return;
   T d[Q];
 #pragma unroll
   for (int s = 0; s < Q; s++) d[s] = ldn<NT>(f + pidx<Q, LAYOUT>(n, Lattice<Q>::opp(s), i));
@@ -77,19 +192,19 @@ __global__ void __launch_bounds__(256)
 }
 
 // AA odd: src/kernels/KernelAA_SOA_Base.cpp:257-342 (AOS: KernelAA_AOS_Base.cpp:258-342)
-template <int Q, typename T, int LAYOUT, bool NT>
+template <int Q, typename T, int LAYOUT, bool NT, bool COMP>
 __global__ void __launch_bounds__(256)
-    k_sparse_aa_odd(T* __restrict__ f, const int32_t* __restrict__ adj, int64_t n, int64_t start,
-                    int64_t count, double omega, T F0, T F1, T F2, uint32_t group) {
-  const int64_t i = start + node_block(group) * blockDim.x + threadIdx.x;
-  if (i >= start + count) return;
-  T d[Q];
+    k_sparse_aa_odd(T* __restrict__ f, AdjTables adj, int64_t n, int64_t start, int64_t count,
+                    double omega, T F0, T F1, T F2, uint32_t group) {
+  const int64_t i = node_of(start, group);
+  const bool active = i >= start && i < start + count;
+  if (COMP ? i / kGroup >= adj.groups : !active) return;
   int32_t loc[Q];
+  neighbour_slots<Q, LAYOUT, NT, COMP>(adj, n, i, active, loc);
+  if (!active) return;
+  T d[Q];
 #pragma unroll
-  for (int s = 0; s < Q; s++) {
-    loc[s] = ldn<NT>(adj + pidx<Q, LAYOUT>(n, s, i));
-    d[s] = f[loc[s]];
-  }
+  for (int s = 0; s < Q; s++) d[s] = f[loc[s]];
   const T F[3] = {F0, F1, F2};
   collide_ref<Q, T, false>(d, d, omega, F, 0.0);
 #pragma unroll
@@ -97,33 +212,54 @@ __global__ void __launch_bounds__(256)
 }
 
 // AB push: src/kernels/KernelAB_SOA_Base.cpp:111-186 (AOS: KernelAB_AOS_Base.cpp:108-182)
-template <int Q, typename T, int LAYOUT, bool NT>
+template <int Q, typename T, int LAYOUT, bool NT, bool COMP>
 __global__ void __launch_bounds__(256)
-    k_sparse_ab_push(const T* __restrict__ src, T* __restrict__ tgt,
-                     const int32_t* __restrict__ adj, int64_t n, int64_t start, int64_t count,
-                     double omega, T F0, T F1, T F2, uint32_t group) {
-  const int64_t i = start + node_block(group) * blockDim.x + threadIdx.x;
-  if (i >= start + count) return;
+    k_sparse_ab_push(const T* __restrict__ src, T* __restrict__ tgt, AdjTables adj, int64_t n,
+                     int64_t start, int64_t count, double omega, T F0, T F1, T F2, uint32_t group) {
+  const int64_t i = node_of(start, group);
+  const bool active = i >= start && i < start + count;
+  if (COMP ? i / kGroup >= adj.groups : !active) return;
   T d[Q];
-#pragma unroll
-  for (int s = 0; s < Q; s++) d[s] = ldn<NT>(src + pidx<Q, LAYOUT>(n, s, i));
   const T F[3] = {F0, F1, F2};
-  collide_ref<Q, T, false>(d, d, omega, F, 0.0);
+  if constexpr (COMP) {
+    if (active) {
 #pragma unroll
-  for (int s = 0; s < Q; s++) tgt[ldn<NT>(adj + pidx<Q, LAYOUT>(n, s, i))] = d[s];
+      for (int s = 0; s < Q; s++) d[s] = ldn<NT>(src + pidx<Q, LAYOUT>(n, s, i));
+    }
+    int32_t loc[Q];
+    neighbour_slots<Q, LAYOUT, NT, true>(adj, n, i, active, loc);
+    if (!active) return;
+    collide_ref<Q, T, false>(d, d, omega, F, 0.0);
+#pragma unroll
+    for (int s = 0; s < Q; s++) tgt[loc[s]] = d[s];
+  } else {
+#pragma unroll
+    for (int s = 0; s < Q; s++) d[s] = ldn<NT>(src + pidx<Q, LAYOUT>(n, s, i));
+    collide_ref<Q, T, false>(d, d, omega, F, 0.0);
+#pragma unroll
+    for (int s = 0; s < Q; s++) tgt[ldn<NT>(adj.adj + pidx<Q, LAYOUT>(n, s, i))] = d[s];
+  }
 }
 
 // AB pull: src/kernels/KernelAB_SOA_Pull.cpp:113-194
-template <int Q, typename T, int LAYOUT, bool NT>
+template <int Q, typename T, int LAYOUT, bool NT, bool COMP>
 __global__ void __launch_bounds__(256)
-    k_sparse_ab_pull(const T* __restrict__ src, T* __restrict__ tgt,
-                     const int32_t* __restrict__ adj, int64_t n, int64_t start, int64_t count,
-                     double omega, T F0, T F1, T F2, uint32_t group) {
-  const int64_t i = start + node_block(group) * blockDim.x + threadIdx.x;
-  if (i >= start + count) return;
+    k_sparse_ab_pull(const T* __restrict__ src, T* __restrict__ tgt, AdjTables adj, int64_t n,
+                     int64_t start, int64_t count, double omega, T F0, T F1, T F2, uint32_t group) {
+  const int64_t i = node_of(start, group);
+  const bool active = i >= start && i < start + count;
+  if (COMP ? i / kGroup >= adj.groups : !active) return;
   T d[Q];
+  if constexpr (COMP) {
+    int32_t loc[Q];
+    neighbour_slots<Q, LAYOUT, NT, true>(adj, n, i, active, loc);
+    if (!active) return;
 #pragma unroll
-  for (int s = 0; s < Q; s++) d[s] = src[ldn<NT>(adj + pidx<Q, LAYOUT>(n, s, i))];
+    for (int s = 0; s < Q; s++) d[s] = src[loc[s]];
+  } else {
+#pragma unroll
+    for (int s = 0; s < Q; s++) d[s] = src[ldn<NT>(adj.adj + pidx<Q, LAYOUT>(n, s, i))];
+  }
   const T F[3] = {F0, F1, F2};
   collide_ref<Q, T, false>(d, d, omega, F, 0.0);
 #pragma unroll
@@ -210,6 +346,11 @@ struct lbm_sparse {
   double omega = 1.0;
   double force[3] = {1e-6, 0.0, 0.0};
   int32_t* adj = nullptr;  // device copy of the adjacency
+  uint32_t* code = nullptr;  // the adjacency compressed (AdjTables), in adj's allocation
+  int32_t* table = nullptr;
+  uint32_t* raw = nullptr;
+  int64_t groups = 0;
+  lbm::AdjTables tables() const { return {adj, code, table, raw, groups}; }
   // launch shapes: the AA even step (all node-aligned) and the other steps
   unsigned even_bx = 256, step_bx = 256, push_bx = 256;
   size_t even_lds = 0, step_lds = 0, push_lds = 0;
@@ -232,25 +373,30 @@ struct Shape {
   uint32_t group;  // node_block: 0, or node blocks per XCD run (grid a multiple of 8 group)
 };
 
-#define LBM_SPARSE_KERNEL_FN(name)                                                         \
+#define LBM_SPARSE_KERNEL_FN(fn, name, ...)                                                \
   template <int Q, typename T, int L>                                                      \
-  struct name##_fn {                                                                       \
+  struct fn {                                                                              \
     template <typename... A>                                                               \
     static void launch(Shape sh, bool nt, hipStream_t st, A... a) {                        \
       if (nt)                                                                              \
-        hipLaunchKernelGGL((lbm::name<Q, T, L, true>), dim3(sh.grid), dim3(sh.block),      \
-                           sh.lds, st, a...);                                              \
+        hipLaunchKernelGGL((lbm::name<Q, T, L, true __VA_ARGS__>), dim3(sh.grid),          \
+                           dim3(sh.block), sh.lds, st, a...);                              \
       else                                                                                 \
-        hipLaunchKernelGGL((lbm::name<Q, T, L, false>), dim3(sh.grid), dim3(sh.block),     \
-                           sh.lds, st, a...);                                              \
+        hipLaunchKernelGGL((lbm::name<Q, T, L, false __VA_ARGS__>), dim3(sh.grid),         \
+                           dim3(sh.block), sh.lds, st, a...);                              \
     }                                                                                      \
   };
-LBM_SPARSE_KERNEL_FN(k_sparse_aa_even)
-LBM_SPARSE_KERNEL_FN(k_sparse_aa_odd)
-LBM_SPARSE_KERNEL_FN(k_sparse_ab_push)
-LBM_SPARSE_KERNEL_FN(k_sparse_ab_pull)
-LBM_SPARSE_KERNEL_FN(k_sparse_init_rest)
-LBM_SPARSE_KERNEL_FN(k_sparse_mass_partial)
+#define LBM_COMMA ,
+LBM_SPARSE_KERNEL_FN(k_sparse_aa_even_fn, k_sparse_aa_even)
+LBM_SPARSE_KERNEL_FN(k_sparse_aa_odd_fn, k_sparse_aa_odd, LBM_COMMA true)
+LBM_SPARSE_KERNEL_FN(k_sparse_aa_odd_raw_fn, k_sparse_aa_odd, LBM_COMMA false)
+LBM_SPARSE_KERNEL_FN(k_sparse_ab_push_fn, k_sparse_ab_push, LBM_COMMA true)
+LBM_SPARSE_KERNEL_FN(k_sparse_ab_push_raw_fn, k_sparse_ab_push, LBM_COMMA false)
+LBM_SPARSE_KERNEL_FN(k_sparse_ab_pull_fn, k_sparse_ab_pull, LBM_COMMA true)
+LBM_SPARSE_KERNEL_FN(k_sparse_ab_pull_raw_fn, k_sparse_ab_pull, LBM_COMMA false)
+LBM_SPARSE_KERNEL_FN(k_sparse_init_rest_fn, k_sparse_init_rest)
+LBM_SPARSE_KERNEL_FN(k_sparse_mass_partial_fn, k_sparse_mass_partial)
+#undef LBM_COMMA
 #undef LBM_SPARSE_KERNEL_FN
 
 template <template <int, typename, int> class K, typename T, typename... A>
@@ -262,6 +408,14 @@ void launch_qt(const lbm_sparse* h, Shape sh, A... a) {
     if (h->layout == LBM_LAYOUT_SOA) K<27, T, LBM_LAYOUT_SOA>::launch(sh, h->nt, h->stream, a...);
     else K<27, T, LBM_LAYOUT_AOS>::launch(sh, h->nt, h->stream, a...);
   }
+}
+
+// A kernel that reads the adjacency: COMP where it is compressed, RAW otherwise.
+template <template <int, typename, int> class COMP, template <int, typename, int> class RAW,
+          typename T, typename... A>
+void launch_adj(const lbm_sparse* h, Shape sh, A... a) {
+  if (h->code) launch_qt<COMP, T>(h, sh, a...);
+  else launch_qt<RAW, T>(h, sh, a...);
 }
 
 // Node blocks per XCD run (node_block).  Measured on the reference's decks
@@ -288,10 +442,12 @@ Shape make_shape(const lbm_sparse* h, int64_t count, unsigned bx, size_t lds, bo
   const unsigned span = 8 * g;
   return {(nb + span - 1) / span * span, bx, lds, g};
 }
-Shape even_shape(const lbm_sparse* h, int64_t count) {
-  return make_shape(h, count, h->even_bx, h->even_lds, false);
+// (node blocks start at the multiple of 64 at or before `start`, node_of)
+Shape even_shape(const lbm_sparse* h, int64_t start, int64_t count) {
+  return make_shape(h, count + (start & 63), h->even_bx, h->even_lds, false);
 }
-Shape step_shape(const lbm_sparse* h, int64_t count, bool push = false) {
+Shape step_shape(const lbm_sparse* h, int64_t start, int64_t count, bool push = false) {
+  count += start & 63;
   return push ? make_shape(h, count, h->push_bx, h->push_lds, true)
               : make_shape(h, count, h->step_bx, h->step_lds, false);
 }
@@ -328,6 +484,63 @@ void set_shapes(lbm_sparse* h) {
   h->step_lds = lds_for(env_int("LBM_SPARSE_BLOCKS_PER_CU", 0));
   h->push_bx = clamp_bx(env_int("LBM_SPARSE_BLOCK_X", big ? 128 : 256));
   h->push_lds = lds_for(env_int("LBM_SPARSE_BLOCKS_PER_CU", big ? 4 : 0));
+}
+
+template <int Q>
+void launch_compress(const lbm_sparse* h) {
+  const dim3 g((unsigned)h->groups), b(kGroup);
+  if (h->layout == LBM_LAYOUT_SOA)
+    hipLaunchKernelGGL((k_sparse_compress<Q, LBM_LAYOUT_SOA>), g, b, 0, h->stream, h->adj, h->code,
+                       h->table, h->raw, h->n);
+  else
+    hipLaunchKernelGGL((k_sparse_compress<Q, LBM_LAYOUT_AOS>), g, b, 0, h->stream, h->adj, h->code,
+                       h->table, h->raw, h->n);
+}
+
+// Device copy of the adjacency and its compressed form.  Waits for both: later
+// steps may run on another stream.
+lbm_status upload_adjacency(lbm_sparse* h, const int32_t* adjacency) {
+  const size_t nq = (size_t)h->n * h->q;
+  h->groups = (h->n + kGroup - 1) / kGroup;
+  // Short lists are bound by latency and one more dependent load costs more than
+  // the traffic it saves.  Reference pipes, D3Q19, caller's table / compressed,
+  // us per step: FP64 103k nodes (simulationSize 1.75) push 8.0 / 7.9, pull 8.2 /
+  // 8.0, 153k (2) AA 9.6 / 9.2, push 10.5 / 10.4, pull 11.4 / 10.7, 1.15M (4) 66.6
+  // / 54.3, 74.6 / 64.9, 87.2 / 76.6; FP32 153k push 7.2 / 7.5, 296k (2.5) push
+  // 12.6 / 11.4, pull 12.6 / 11.5.  LBM_SPARSE_COMPRESS=0|1 overrides.
+  const char* env = std::getenv("LBM_SPARSE_COMPRESS");
+  const size_t esize = h->storage == LBM_STORE_F64 ? 8 : 4;
+  const bool compress = env ? env[0] != '0' : h->n * esize >= 1100000;
+  // one allocation: the caller's table, codes, tables of distances, raw flags
+  const size_t words = h->q == 19 ? code_words<19>() : code_words<27>();
+  auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t adj_b = pad(sizeof(int32_t) * nq),
+               code_b = pad(sizeof(uint32_t) * words * h->groups * kGroup),
+               table_b = pad(sizeof(int32_t) * h->groups * h->q * kDeltas),
+               raw_b = pad(sizeof(uint32_t) * h->groups);
+  if (hipMalloc(&h->adj, adj_b + (compress ? code_b + table_b + raw_b : 0)) != hipSuccess) {
+    h->adj = nullptr;
+    set_error("lbm_sparse_create: hipMalloc of the adjacency failed");
+    return LBM_ERR_OOM;
+  }
+  if (compress) {
+    char* p = (char*)h->adj + adj_b;
+    h->code = (uint32_t*)p;
+    h->table = (int32_t*)(p + code_b);
+    h->raw = (uint32_t*)(p + code_b + table_b);
+  }
+  hipError_t e = hipMemcpy(h->adj, adjacency, sizeof(int32_t) * nq, hipMemcpyHostToDevice);
+  if (e == hipSuccess && compress) {
+    if (h->q == 19) launch_compress<19>(h);
+    else launch_compress<27>(h);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  }
+  if (e != hipSuccess) {
+    set_error("lbm_sparse_create: adjacency copy failed: %s", hipGetErrorString(e));
+    return LBM_ERR_HIP;
+  }
+  return LBM_OK;
 }
 
 lbm_status check_range(const lbm_sparse* h, int64_t start, int64_t count) {
@@ -410,7 +623,11 @@ lbm_status lbm_sparse_create(const lbm_sparse_config* cfg, lbm_sparse** out) {
   LBM_REQUIRE(cfg->n_fluid * cfg->q < ((int64_t)1 << 31), LBM_ERR_ARG,
               "lbm_sparse_create: n_fluid * q must fit the int32 adjacency");
   const int64_t nq = cfg->n_fluid * cfg->q;
-  for (int64_t k = 0; k < nq; k++)
+  // every entry in [0, nq): first without a branch (negative ones wrap to large
+  // ones), then, if one is not, which
+  uint32_t bad = 0;
+  for (int64_t k = 0; k < nq; k++) bad |= (uint32_t)cfg->adjacency[k] >= (uint32_t)nq;
+  for (int64_t k = 0; bad && k < nq; k++)
     LBM_REQUIRE(cfg->adjacency[k] >= 0 && cfg->adjacency[k] < nq, LBM_ERR_ARG,
                 "lbm_sparse_create: adjacency[%lld] = %d outside [0, %lld)", (long long)k,
                 cfg->adjacency[k], (long long)nq);
@@ -427,21 +644,14 @@ lbm_status lbm_sparse_create(const lbm_sparse_config* cfg, lbm_sparse** out) {
     const char* e = std::getenv("LBM_SPARSE_XCD");
     h->xcd_env = e ? std::max(0, std::min(4096, std::atoi(e))) : -1;
   }
-  if (hipMalloc(&h->adj, sizeof(int32_t) * nq) != hipSuccess) {
+  if (lbm_status st = upload_adjacency(h, cfg->adjacency)) {
+    if (h->adj) (void)hipFree(h->adj);
     delete h;
-    set_error("lbm_sparse_create: hipMalloc of the adjacency failed");
-    return LBM_ERR_OOM;
-  }
-  hipError_t e = hipMemcpy(h->adj, cfg->adjacency, sizeof(int32_t) * nq, hipMemcpyHostToDevice);
-  if (e != hipSuccess) {
-    (void)hipFree(h->adj);
-    delete h;
-    set_error("lbm_sparse_create: adjacency copy failed: %s", hipGetErrorString(e));
-    return LBM_ERR_HIP;
+    return st;
   }
   double* scr = nullptr;  // set-up of lbm_sparse_mass_noalloc's scratch on this device
   if (lbm_status st = scratch_on_current_device(&scr)) {
-    (void)hipFree(h->adj);
+    if (h->adj) (void)hipFree(h->adj);
     delete h;
     return st;
   }
@@ -462,7 +672,7 @@ lbm_status lbm_sparse_aa_even(lbm_sparse* h, void* dstrb, int64_t start, int64_t
   LBM_REQUIRE(h && dstrb, LBM_ERR_ARG, "lbm_sparse_aa_even: null pointer");
   if (lbm_status st = check_range(h, start, count)) return st;
   if (count == 0) return LBM_OK;
-  const Shape g = even_shape(h, count);
+  const Shape g = even_shape(h, start, count);
   if (h->storage == LBM_STORE_F64)
     launch_qt<k_sparse_aa_even_fn, double>(h, g, (double*)dstrb, h->n, start, count, h->omega,
                                           h->force[0], h->force[1], h->force[2], g.group);
@@ -480,13 +690,13 @@ lbm_status lbm_sparse_aa_odd(lbm_sparse* h, void* dstrb, int64_t start, int64_t 
               "lbm_sparse_aa_odd: AA needs the x - c_s adjacency (adjacency_mode 1)");
   if (lbm_status st = check_range(h, start, count)) return st;
   if (count == 0) return LBM_OK;
-  const Shape g = step_shape(h, count);
+  const Shape g = step_shape(h, start, count);
   if (h->storage == LBM_STORE_F64)
-    launch_qt<k_sparse_aa_odd_fn, double>(h, g, (double*)dstrb, (const int32_t*)h->adj, h->n,
+    launch_adj<k_sparse_aa_odd_fn, k_sparse_aa_odd_raw_fn, double>(h, g, (double*)dstrb, h->tables(), h->n,
                                          start, count, h->omega, h->force[0], h->force[1],
                                          h->force[2], g.group);
   else
-    launch_qt<k_sparse_aa_odd_fn, float>(h, g, (float*)dstrb, (const int32_t*)h->adj, h->n, start,
+    launch_adj<k_sparse_aa_odd_fn, k_sparse_aa_odd_raw_fn, float>(h, g, (float*)dstrb, h->tables(), h->n, start,
                                         count, h->omega, (float)h->force[0], (float)h->force[1],
                                         (float)h->force[2], g.group);
   LBM_LAUNCH_CHECK();
@@ -503,24 +713,24 @@ lbm_status lbm_sparse_ab(lbm_sparse* h, const void* src, void* tgt, int64_t star
               "lbm_sparse_ab: the reference has no AOS pull kernel");
   if (lbm_status st = check_range(h, start, count)) return st;
   if (count == 0) return LBM_OK;
-  const Shape g = step_shape(h, count, !pull);
-  const int32_t* adj = h->adj;
+  const Shape g = step_shape(h, start, count, !pull);
+  const AdjTables adj = h->tables();
   if (h->storage == LBM_STORE_F64) {
     if (pull)
-      launch_qt<k_sparse_ab_pull_fn, double>(h, g, (const double*)src, (double*)tgt, adj, h->n,
+      launch_adj<k_sparse_ab_pull_fn, k_sparse_ab_pull_raw_fn, double>(h, g, (const double*)src, (double*)tgt, adj, h->n,
                                             start, count, h->omega, h->force[0], h->force[1],
                                             h->force[2], g.group);
     else
-      launch_qt<k_sparse_ab_push_fn, double>(h, g, (const double*)src, (double*)tgt, adj, h->n,
+      launch_adj<k_sparse_ab_push_fn, k_sparse_ab_push_raw_fn, double>(h, g, (const double*)src, (double*)tgt, adj, h->n,
                                             start, count, h->omega, h->force[0], h->force[1],
                                             h->force[2], g.group);
   } else {
     const float F0 = (float)h->force[0], F1 = (float)h->force[1], F2 = (float)h->force[2];
     if (pull)
-      launch_qt<k_sparse_ab_pull_fn, float>(h, g, (const float*)src, (float*)tgt, adj, h->n,
+      launch_adj<k_sparse_ab_pull_fn, k_sparse_ab_pull_raw_fn, float>(h, g, (const float*)src, (float*)tgt, adj, h->n,
                                            start, count, h->omega, F0, F1, F2, g.group);
     else
-      launch_qt<k_sparse_ab_push_fn, float>(h, g, (const float*)src, (float*)tgt, adj, h->n,
+      launch_adj<k_sparse_ab_push_fn, k_sparse_ab_push_raw_fn, float>(h, g, (const float*)src, (float*)tgt, adj, h->n,
                                            start, count, h->omega, F0, F1, F2, g.group);
   }
   LBM_LAUNCH_CHECK();
