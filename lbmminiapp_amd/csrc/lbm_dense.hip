@@ -10,6 +10,8 @@
 //   AB push         f_s(x) in slot s at x of the current array
 //   AB pull         the current array holds post-collision values; f_s(x) is gathered
 //                   like the AA odd case (src/kernels/KernelAB_SOA_Pull.cpp:139-140)
+//   through walls   AB pull with f_s(x) in slot s at x - c_s also where x - c_s is solid
+//                   or outside (wrapped)
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -19,7 +21,7 @@
 
 namespace lbm {
 
-enum CanonMode { C_LOCAL = 0, C_OPP = 1, C_GATHER = 2 };
+enum CanonMode { C_LOCAL = 0, C_OPP = 1, C_GATHER = 2, C_WALL = 3 };
 
 // storage cell of cell = (x, y, z): on interleaved rows element x of the row
 // sits at position ir_pos(x)
@@ -34,7 +36,8 @@ __device__ __forceinline__ int64_t canon_index(int mode, int s, int64_t cell, in
   const int64_t n = a.ncell;
   const int o = Lattice<Q>::opp(s);
   if (mode == C_LOCAL) return slot<Q, LAYOUT>(n, s, store_cell(a, cell, x));
-  if (mode == C_OPP || ((lk >> o) & 1u)) return slot<Q, LAYOUT>(n, o, store_cell(a, cell, x));
+  if (mode == C_OPP || (mode == C_GATHER && ((lk >> o) & 1u)))
+    return slot<Q, LAYOUT>(n, o, store_cell(a, cell, x));
   const int cx = Lattice<Q>::c(s, 0);
   return slot<Q, LAYOUT>(
       n, s,
@@ -88,7 +91,7 @@ __global__ void __launch_bounds__(256)
 // across the periodic x boundary (canonical = stored + sign * w_s * djump).
 template <int Q>
 __device__ __forceinline__ int canon_jump_sign(int mode, int s, int x, uint32_t lk, int nx) {
-  if (mode != C_GATHER || ((lk >> Lattice<Q>::opp(s)) & 1u)) return 0;
+  if (mode < C_GATHER || ((lk >> Lattice<Q>::opp(s)) & 1u)) return 0;
   return gather_crossing(Lattice<Q>::c(s, 0), x, nx);
 }
 
@@ -228,11 +231,12 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------- mass
-// Sum over every fluid cell of its Q stored values (any state convention is a
-// permutation of the canonical populations over the fluid slots).
+// Sum over every fluid cell of its Q stored values (any state convention but
+// through walls is a permutation of the canonical populations over the fluid
+// slots; there the values are gathered).
 template <int Q, int STORE, int LAYOUT>
 __global__ void __launch_bounds__(256)
-    k_mass_partial(const void* fv, DenseArgs a, double* partial) {
+    k_mass_partial(const void* fv, DenseArgs a, int mode, double* partial) {
   const auto* f = static_cast<const typename Storage<STORE>::T*>(fv);
   __shared__ double red[256];
   double acc = 0.0;
@@ -240,6 +244,15 @@ __global__ void __launch_bounds__(256)
   for (int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; cell < a.ncell;
        cell += stride) {
     if (a.links && (a.links[cell] & SOLID_BIT)) continue;
+    if (mode == C_WALL) {
+      const int64_t row = cell / a.nx;
+      const int x = (int)(cell - row * a.nx), y = (int)(row % a.ny), z = (int)(row / a.ny);
+      const Offsets off(x, y, z, a.nx, a.ny, a.nz);
+      for (int s = 0; s < Q; s++)
+        acc += to_f<STORE>(ld<STORE>(f, canon_index<Q, LAYOUT>(mode, s, cell, x, 0u, off, a), a.inv_scale),
+                           Lattice<Q>::w(s));
+      continue;
+    }
     for (int s = 0; s < Q; s++)
       acc += to_f<STORE>(ld<STORE>(f, slot<Q, LAYOUT>(a.ncell, s, cell), a.inv_scale),
                          Lattice<Q>::w(s));
@@ -439,7 +452,7 @@ void set_launch_shapes(lbm_dense* h) {
 // state convention of the current array
 int canon_mode(const lbm_dense* h) {
   if (h->pattern == LBM_PATTERN_AA) return (h->t % 2 == 0) ? C_OPP : C_GATHER;
-  return h->pull ? C_GATHER : C_LOCAL;
+  return h->walls ? C_WALL : (h->pull ? C_GATHER : C_LOCAL);
 }
 
 // kernels with the Guo forcing terms: a nonzero force, or the policy set at create
@@ -587,7 +600,8 @@ lbm_status enqueue_steps(lbm_dense* h, int nsteps) {
     if (h->pattern == LBM_PATTERN_AA) {
       st = launch_kind(h, (h->t % 2 == 0) ? K_AA_EVEN : K_AA_ODD, h->f[0], h->f[0]);
     } else {
-      st = launch_kind(h, h->pull ? K_AB_PULL : K_AB_PUSH, h->f[h->cur], h->f[1 - h->cur]);
+      st = launch_kind(h, h->walls ? K_AB_WALL : (h->pull ? K_AB_PULL : K_AB_PUSH), h->f[h->cur],
+                       h->f[1 - h->cur]);
       h->cur = 1 - h->cur;
     }
     if (st != LBM_OK) return st;
@@ -656,9 +670,9 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
   return p;
 }
 
-// Two steps per launch (lbm_dense_pair.hpp) on unmasked periodic SOA boxes in
-// FP64 and FP32 deviations, without per-cell fields or a pressure drop.  Default
-// from 20,000 cells on; below, the march along z is a longer chain than two
+// Two steps per launch (lbm_dense_pair.hpp) on SOA boxes in FP64 and FP32
+// deviations, without per-cell fields, and with a pressure drop only where there
+// is a mask.  Default from 20,000 cells on; below, the march along z is a longer chain than two
 // launches (us per step, one step / two steps per launch, D3Q19 FP64: 16^3 3.9 /
 // 4.6, 128 x 16 x 8 3.8 / 5.4, 24^3 5.0 / 4.8, 28^3 6.3 / 5.0, 12 x 12 x 200
 // 11.6 / 7.2; every larger size measured gained).  LBM_DENSE_PAIR=0|1 overrides;
@@ -666,22 +680,31 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
 // h->pair_args, and the cache policy: stores stream past the caches when both
 // arrays exceed 320 MiB (100^3 FP64, 290 MiB: 44.0 us cached / 44.7 streaming;
 // 112^3, 408 MiB: 54.4 / 52.9; 120^3 FP32, 250 MiB: 34.4 / 39.8).
-void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links) {
+// Masked boxes gain about 1.2x, so they take pairs only where the tiles waste
+// less than 15% of that against the one-step kernels: tile rows past the box,
+// lanes past the end of narrow rows, and rows that are solid all along, which
+// the one-step kernels skip (`live`: the share of rows that are not).  The
+// reference's pipe, 20% of such rows, loses: simulationSize 2 12.5 / 14.4 us per
+// step, 4 59.5 / 74.7.  An AA box whose array fits the memory-side cache where
+// two do not keeps its one array (100^3 porous D3Q19 FP64 52.8 / 55.8).
+void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, double live) {
   const char* e = std::getenv("LBM_DENSE_PAIR");
   bool on = h->ncell >= 20000;
   for (const char* v : {"LBM_DENSE_IROWS", "LBM_DENSE_ODD_SEG", "LBM_DENSE_SLAB_PLANES",
-                        "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS"})
+                        "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS", "LBM_DENSE_PUSH_GATHER",
+                        "LBM_DENSE_FILL_SOLID"})
     on = on && !std::getenv(v);
   if (e) on = e[0] != '0';
   const size_t plane_bytes = (size_t)h->nx * h->ny * h->esize;
-  if (!on || need_links || h->layout != LBM_LAYOUT_SOA || cfg->tau || cfg->gamma ||
-      cfg->density_jump_x != 0.0 || plane_bytes > UINT32_MAX)
+  if (!on || h->layout != LBM_LAYOUT_SOA || cfg->tau || cfg->gamma ||
+      (!need_links && cfg->density_jump_x != 0.0) || plane_bytes >= UINT32_MAX)
     return;
   const bool force = cfg->force[0] != 0.0 || cfg->force[1] != 0.0 || cfg->force[2] != 0.0;
   bool nt = h->nt;
   if (!std::getenv("LBM_DENSE_NT"))
     nt = 2 * (size_t)h->ncell * h->q * h->esize > ((size_t)320 << 20);
-  const auto pick = h->q == 19 ? pick_pair19 : pick_pair27;
+  const auto pick = h->q == 19 ? (need_links ? pick_pair19_mask : pick_pair19)
+                               : (need_links ? pick_pair27_mask : pick_pair27);
   auto slots = [](const PairKernel& k) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -699,6 +722,13 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links) {
     if (s <= 0) return;
     const PairArgs p = plan_pair(k, h->nx, h->ny, h->nz, s);
     if ((int64_t)p.ntx * p.nty * p.nch >= ((int64_t)1 << 28)) return;
+    if (need_links && !e) {
+      const size_t cache = (size_t)256 << 20, one = (size_t)h->ncell * h->q * h->esize;
+      const double rows = (double)h->ny / (p.nty * k.ty),
+                   lanes = (double)((h->nx + 63) / 64 * 64) / (p.ntx * k.w);
+      if (live * rows * lanes < 0.85) return;
+      if (h->pattern == LBM_PATTERN_AA && one <= cache && 2 * one > cache) return;
+    }
     h->pair = k;
     h->pair_args = p;
     if ((int64_t)p.ntx * p.nty * h->nz > s) return;
@@ -743,10 +773,17 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   set_launch_shapes(h);  // after ncell and esize: the cache policy depends on the footprint
   // fluid count (host mask)
   h->nfluid = h->ncell;
+  double live = 1.0;  // share of x-rows with fluid cells
   if (cfg->solid) {
-    int64_t ns = 0;
-    for (int64_t c = 0; c < h->ncell; c++) ns += cfg->solid[c] != 0;
+    int64_t ns = 0, dead = 0;
+    for (int64_t c = 0; c < h->ncell; c += h->nx) {
+      int64_t n = 0;
+      for (int x = 0; x < h->nx; x++) n += cfg->solid[c + x] != 0;
+      ns += n;
+      dead += n == h->nx;
+    }
     h->nfluid = h->ncell - ns;
+    live = 1.0 - (double)dead / ((double)h->ny * h->nz);
   }
   const bool need_links =
       cfg->solid != nullptr || !h->periodic[0] || !h->periodic[1] || !h->periodic[2];
@@ -755,7 +792,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   // box they take a second population array, so only while both fit easily: a
   // quarter of the GPU's memory, and half of what is free (512^3 D3Q19 FP64:
   // 41 of 288 GB).  Larger boxes, and a GPU that is nearly full, step in place.
-  if (pair_ok) choose_pair(h, cfg, need_links);
+  if (pair_ok) choose_pair(h, cfg, need_links, live);
   const bool aa_as_pairs = h->pair.launch && h->pattern == LBM_PATTERN_AA;
   if (aa_as_pairs) {
     size_t room = 0, total = 0;
@@ -766,6 +803,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   if (h->pair.launch) {
     h->pattern = LBM_PATTERN_AB;
     h->pull = 1;
+    h->walls = need_links;
   }
   // Interleaved rows (lbm_dense_kernels.hpp) for AA on unmasked periodic SOA
   // boxes whose rows are whole 64-element blocks: the odd step then makes only
@@ -1203,7 +1241,7 @@ lbm_status lbm_dense_moments(lbm_dense* h, double* rho, double* u) {
 lbm_status lbm_dense_mass(lbm_dense* h, double* mass) {
   LBM_REQUIRE(h && mass, LBM_ERR_ARG, "lbm_dense_mass: null pointer");
   launch_util<k_mass_partial_u>(h->q, h->storage, h->layout, dim3(h->npartial), dim3(256),
-                                h->stream, (const void*)h->f[h->cur], h->args, h->partial);
+                                h->stream, (const void*)h->f[h->cur], h->args, canon_mode(h), h->partial);
   LBM_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, h->stream, (const double*)h->partial,
                      h->npartial, h->partial + h->npartial);

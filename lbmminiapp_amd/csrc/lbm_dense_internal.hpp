@@ -23,6 +23,7 @@ struct lbm_dense {
   size_t odd_ir_lds = 0;
   lbm::PairKernel pair{};  // two time steps per launch (k_dense_pair); launch == nullptr: off
   lbm::PairArgs pair_args{};
+  bool walls = false;        // state through walls (K_AB_WALL), masked boxes in pairs
   bool own_capture = false;  // lbm_dense_graph_create is recording
   int64_t ncell = 0, nfluid = 0, t = 0;
   size_t esize = 8;

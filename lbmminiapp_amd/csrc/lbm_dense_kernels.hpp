@@ -27,6 +27,13 @@
 //            (src/kernels/KernelAB_SOA_Base.cpp:111-186)
 //   AB_PULL  read slot s at x - c_s [slot opp(s) at x], write slot s at x
 //            (src/kernels/KernelAB_SOA_Pull.cpp:113-194)
+//   AB_WALL  read slot s at x - c_s, write slot s at x [slot opp(s) at x + c_s]:
+//            AB_PULL with the bounce-back moved from the gather to the store.
+//            A result that a blocked link sends back goes where the same cell's
+//            next gather looks for it, into the solid cell's slot (or that of
+//            the cell at the other end of a non-periodic box, whose own result
+//            in that direction leaves the box too): every slot still has one
+//            writer and one reader, and the gather reads whole rows.
 // AA touches the same Q slots for reading and writing, so it runs in place
 // with no inter-workgroup synchronisation.
 //
@@ -52,7 +59,9 @@ namespace lbm {
 constexpr uint32_t SOLID_BIT = 1u << 31;
 
 // K_AA_ODD_IR: the AA odd step on interleaved rows
-enum DenseKind { K_AA_EVEN = 0, K_AA_ODD = 1, K_AB_PUSH = 2, K_AB_PULL = 3, K_AA_ODD_IR = 4 };
+enum DenseKind {
+  K_AA_EVEN = 0, K_AA_ODD = 1, K_AB_PUSH = 2, K_AB_PULL = 3, K_AA_ODD_IR = 4, K_AB_WALL = 5
+};
 
 // Interleaved rows: position of x, x at position p, and the position of
 // x + d (d in {-1, 0, 1}, periodic) from the position p of x.
@@ -308,7 +317,9 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
     k_dense(const typename Storage<STORE>::T* f0, typename Storage<STORE>::T* f1, DenseArgs a) {
   using C = typename Storage<STORE>::C;
   constexpr bool IR = KIND == K_AA_ODD_IR;
+  constexpr bool WALL = KIND == K_AB_WALL;
   static_assert(!IR || (!MASK && LAYOUT == LBM_LAYOUT_SOA), "interleaved rows: unmasked SOA only");
+  static_assert(!WALL || (MASK && LAYOUT == LBM_LAYOUT_SOA), "through-wall slots: masked SOA only");
   // x: the thread's row position (on interleaved rows, a.xk != 0, element xr
   // of the row).  Interleaved rows make every x-shifted access one aligned
   // block as well (see the file comment).
@@ -379,11 +390,12 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
         idx = slot<Q, LAYOUT>(n, s, cell);
       } else {
         aligned = cx == 0 || irows;
-        if (MASK && ((lk >> o) & 1u)) {
+        const bool bb = MASK && ((lk >> o) & 1u);
+        if (bb && !WALL) {
           idx = slot<Q, LAYOUT>(n, o, cell);
         } else {
           idx = slot<Q, LAYOUT>(n, s, cell + off.at(-cx, -cy, -cz));
-          cross = gather_crossing(cx, xr, a.nx);
+          cross = bb ? 0 : gather_crossing(cx, xr, a.nx);
         }
       }
       if (aligned && LAYOUT == LBM_LAYOUT_SOA) d[s] = ld_s<STORE, NT>(f0, idx, a.inv_scale);
@@ -429,6 +441,14 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
     const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
     if constexpr (KIND == K_AA_EVEN || KIND == K_AB_PULL) {
       put(slot<Q, LAYOUT>(n, s, cell), solid ? C(0) : d[s], true);
+    } else if constexpr (WALL) {
+      // Slot s at x belongs to the cell beyond a blocked link where that cell is
+      // fluid: a fluid x stores it unless the link leaves the box (a copy nobody
+      // reads completes the line), a solid x stores a zero unless its neighbour
+      // there is fluid, or may be (links that leave the box).
+      const bool bb = (lk >> s) & 1u, out = leaves_box(a, xr, y, z, cx, cy, cz);
+      if (solid ? bb && !out : !(bb && out)) put(slot<Q, LAYOUT>(n, s, cell), solid ? C(0) : d[s], true);
+      if (bb && !solid) put(slot<Q, LAYOUT>(n, o, cell + off.at(cx, cy, cz)), d[s], false);
     } else {
       const bool aligned = cx == 0 || irows;
       // streaming target: AA odd writes slot opp(s) at x + c_s, AB push slot s
@@ -880,6 +900,13 @@ DenseLaunchFn pick_kind(int kind, bool mask, bool force) {
     case K_AA_ODD: return pick_flags<Q, STORE, LAYOUT, K_AA_ODD, NT>(mask, force);
     case K_AB_PUSH: return pick_flags<Q, STORE, LAYOUT, K_AB_PUSH, NT>(mask, force);
     case K_AB_PULL: return pick_flags<Q, STORE, LAYOUT, K_AB_PULL, NT>(mask, force);
+    case K_AB_WALL:
+      if constexpr (LAYOUT == LBM_LAYOUT_SOA) {
+        if (!mask) return nullptr;
+        return force ? launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, true, NT>
+                     : launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, false, NT>;
+      }
+      return nullptr;
     case K_AA_ODD_IR:
       if constexpr (LAYOUT == LBM_LAYOUT_SOA) {
         if (mask) return nullptr;

@@ -38,10 +38,20 @@
 // Work items go to the XCDs in contiguous runs (x fastest, then y, then chunks),
 // so that the tiles whose rings overlap share an L2.
 //
+// Masked boxes (MASK) hold their state through walls (K_AB_WALL): the gather
+// needs no links, so loads stay whole rows, and the stores put what a blocked
+// link sends back where the next gather looks for it.  Between the two steps a
+// blocked link takes the cell's own result instead of the neighbour's, from its
+// own LDS position or register.  Per-lane addresses chosen by link in the gather
+// made the pairs slower than single steps (384 x 250 x 260 porous, D3Q19 FP32:
+// 968 us per step; now 618, single steps 772).
+//
 // Measured, ms per step, one-step kernels -> pairs (tile as choose_pair takes it):
 //   D3Q19 FP64 512^3 7.15 -> 4.10   256^3 0.912 -> 0.493   128^3 0.110 -> 0.067
 //   D3Q19 FP32 512^3 3.42 -> 2.38   256^3 0.409 -> 0.266
 //   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 384^3 2.40 -> 1.51
+//   channel with 5% spheres 256^3 D3Q19 FP64 0.930 -> 0.778   FP32 0.450 -> 0.338
+//   porous 384 x 250 x 260, 35% solid, D3Q19 FP64 1.37 -> 1.14   FP32 0.772 -> 0.618
 #pragma once
 #include "lbm_dense_kernels.hpp"
 
@@ -88,7 +98,30 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t v) {
   return v;
 }
 
-template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+// Directions with a component of the given sign along axis d, as link bits.
+template <int Q>
+__host__ __device__ constexpr uint32_t dirs_along(int d, int sign) {
+  uint32_t m = 0;
+  for (int s = 0; s < Q; s++) m |= (uint32_t)(Lattice<Q>::c(s, d) == sign) << s;
+  return m;
+}
+
+// Store of one element at a lane's byte offset from a uniform base, dropped by
+// the buffer's range check where `keep` is false: no branch around the store.
+template <bool NT, typename T>
+__device__ __forceinline__ void buffer_put(void* base, uint32_t bytes, uint32_t off, bool keep, T v) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)scalar_base(base), 0, bytes, 0x00020000);
+  const uint32_t o = keep ? off : 0xffffffffu;
+  constexpr int aux = NT ? 2 : 0;  // nt
+  if constexpr (sizeof(T) == 8) {
+    typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r, o, 0, aux);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, o, 0, aux);
+  }
+}
+
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
 __global__ void __launch_bounds__((pair_threads<W, TY>()))
     k_dense_pair(const typename Storage<STORE>::T* __restrict__ f0,
                  typename Storage<STORE>::T* __restrict__ f1, DenseArgs a, PairArgs pa) {
@@ -140,22 +173,56 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
   const int64_t n = a.ncell, plane = (int64_t)a.nx * a.ny;
   const double F[3] = {a.F0, a.F1, a.F2};
 
+  uint32_t lk = 0, lk_next = 0, lk_prev = 0;  // links of planes p, p + 1, p - 1
+  auto load_links = [&](int p) -> uint32_t {
+    if constexpr (MASK) {
+      const auto base = scalar_base(a.links + plane * wrap1(p < ze ? p : ze, a.nz));
+      return *(global_ptr<const uint32_t>)(base + lane_offset(off[1][1] / (uint32_t)sizeof(T) * 4u));
+    }
+    return 0u;
+  };
+  // a population that crossed the periodic x boundary along an open link
+  auto jump = [&](C(&d)[Q], uint32_t k) {
+    if (MASK && a.djump != 0.0) {
+#pragma unroll
+      for (int s = 0; s < Q; s++) {
+        const int cx = Lattice<Q>::c(s, 0);
+        const bool wall = (k >> Lattice<Q>::opp(s)) & 1u;
+        if (cx != 0) d[s] = with_jump<Q>(d[s], wall ? 0 : gather_crossing(cx, x, a.nx), s, a.djump);
+      }
+    }
+  };
   auto collide = [&](C* d) {
-    collide_cell<Q, STORE, FORCE, false>(d, a.omega, F, nullptr, 0);
+    double G[3] = {F[0], F[1], F[2]};
+    // masked FP64 keeps no products with the force in registers across the loop
+    if constexpr (MASK && FORCE && STORE == LBM_STORE_F64)
+      asm volatile("" : "+v"(G[0]), "+v"(G[1]), "+v"(G[2]));
+    collide_cell<Q, STORE, FORCE, false>(d, a.omega, G, nullptr, 0);
+  };
+  // ncell, opaque: the Q slot offsets are summed up again at each use rather than
+  // kept in (and spilled from) scalar registers
+  auto slot_stride = [&]() -> int64_t {
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)n >> 32)) << 32) |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)n));
   };
   // gathers the populations of plane p (past the chunk: of its last halo plane again)
   auto load_plane = [&](int p, C(&f)[Q]) {
     const int z = wrap1(p < ze ? p : ze, a.nz);
-    const int zz[3] = {wrap1(z + 1, a.nz), z, wrap1(z - 1, a.nz)};  // source of cz = -1, 0, 1
+    const T* src[3] = {f0 + plane * wrap1(z + 1, a.nz), f0 + plane * z,
+                       f0 + plane * wrap1(z - 1, a.nz)};  // plane of cz = -1, 0, 1
+    const int64_t step = slot_stride();
+    int64_t at = 0;
 #pragma unroll
     for (int s = 0; s < Q; s++) {
-      const auto base = scalar_base(f0 + (n * s + plane * zz[Lattice<Q>::c(s, 2) + 1]));
+      const auto base = scalar_base(src[Lattice<Q>::c(s, 2) + 1] + at);
+      at += step;
       f[s] = *(global_ptr<const T>)(
           base + lane_offset(off[Lattice<Q>::c(s, 0) + 1][Lattice<Q>::c(s, 1) + 1]));
     }
   };
   C own[3];  // the first step's results that stay in the lane, by cz + 1
   auto first_step = [&](C(&f)[Q]) {
+    jump(f, lk);
     collide(f);
 #pragma unroll
     for (int s = 0; s < Q; s++) {
@@ -167,42 +234,101 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
   };
 
   C f[Q];
+  lk = load_links(zc - 1);
+  lk_next = load_links(zc);
   load_plane(zc - 1, f);
   if (!inner) {
     for (int p = zc - 1; p <= ze; p++) {
       first_step(f);
+      const uint32_t lk_after = load_links(p + 2);
       load_plane(p + 1, f);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();  // LDS holds plane p
       __syncthreads();  // LDS has been read
+      lk = lk_next;
+      lk_next = lk_after;
     }
     return;
   }
 
   // Populations of the second step: h of cz = 0 and cz = 1 for plane p - 1, and
-  // of cz = 1 for plane p (next), by direction.
+  // of cz = 1 for plane p (next), by direction.  Masked, h of cz = -1 is what a
+  // blocked link sends back: the cell's own result in the opposite direction.
   C h[Q] = {}, next[Q] = {};
+  auto blocked = [&](uint32_t k, int s) { return MASK && ((k >> Lattice<Q>::opp(s)) & 1u); };
   // what the cell receives in direction s from the plane in LDS
-  auto receive = [&](int s) -> C {
+  auto receive = [&](int s, bool wall) -> C {
     const int k = pair_slot<Q>(s);
-    return k < 0 ? own[Lattice<Q>::c(s, 2) + 1]
-                 : lds[k * PL + lo - Lattice<Q>::c(s, 1) * EX - Lattice<Q>::c(s, 0)];
+    if (k < 0) return own[(wall ? -1 : 1) * Lattice<Q>::c(s, 2) + 1];
+    int pos = k * PL + lo - Lattice<Q>::c(s, 1) * EX - Lattice<Q>::c(s, 0);
+    if (wall) pos = pair_slot<Q>(Lattice<Q>::opp(s)) * PL + lo;
+    return lds[pos];
   };
   auto second_step = [&](int z) {
     C d[Q];
 #pragma unroll
-    for (int s = 0; s < Q; s++) d[s] = Lattice<Q>::c(s, 2) < 0 ? receive(s) : h[s];
-    collide(d);
-#pragma unroll
     for (int s = 0; s < Q; s++) {
-      const auto q = (global_ptr<T>)(scalar_base(f1 + (n * s + plane * z)) + lane_offset(off[1][1]));
-      if constexpr (NT) __builtin_nontemporal_store(d[s], q);
-      else *q = d[s];
+      d[s] = h[s];
+      if (Lattice<Q>::c(s, 2) < 0) {
+        const C v = receive(s, false);
+        d[s] = blocked(lk_prev, s) ? h[s] : v;
+      }
+    }
+    jump(d, lk_prev);
+    collide(d);
+    const uint32_t here = off[1][1];
+    if constexpr (!MASK) {
+      T* dst = f1 + plane * z;
+      const int64_t step = slot_stride();
+#pragma unroll
+      for (int s = 0; s < Q; s++) {
+        const auto q = (global_ptr<T>)(scalar_base(dst) + lane_offset(here));
+        dst += step;
+        if constexpr (NT) __builtin_nontemporal_store(d[s], q);
+        else *q = d[s];
+      }
+    } else {
+      // Links that leave the box through a non-periodic face: there the slot
+      // belongs to the cell at the other end.
+      const uint32_t open = a.periodic_bits;
+      uint32_t out = 0;
+      if (!(open & 1u)) out |= (x == 0 ? dirs_along<Q>(0, -1) : 0u) | (x == a.nx - 1 ? dirs_along<Q>(0, 1) : 0u);
+      if (!(open & 2u)) out |= (y == 0 ? dirs_along<Q>(1, -1) : 0u) | (y == a.ny - 1 ? dirs_along<Q>(1, 1) : 0u);
+      if (!(open & 4u)) out |= (z == 0 ? dirs_along<Q>(2, -1) : 0u) | (z == a.nz - 1 ? dirs_along<Q>(2, 1) : 0u);
+      const bool solid = (lk_prev & SOLID_BIT) != 0;
+      const uint32_t wall = solid ? 0u : lk_prev;
+      const uint32_t keep = solid ? (__all(solid) ? 0u : lk_prev & ~out) : ~(lk_prev & out);
+      const uint32_t bytes = (uint32_t)(plane * sizeof(T));
+      // What blocked links send back, then the whole rows: the branches of the
+      // first leave a known number of stores after them.  (The barriers keep the
+      // lane offsets of all 37 stores from being live at once.)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < Q; s++) {
+        const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
+        if ((cx != 0 || cy != 0 || cz != 0) && ((wall >> s) & 1u)) {
+          const auto base = scalar_base(f1 + (n * Lattice<Q>::opp(s) + plane * wrap1(z + cz, a.nz)));
+          *(global_ptr<T>)(base + lane_offset(off[1 - cx][1 - cy])) = d[s];
+        }
+      }
+      T* dst = f1 + plane * z;
+      const int64_t step = slot_stride();
+#pragma unroll
+      for (int s = 0; s < Q; s++) {
+        buffer_put<NT>(dst + step * s, bytes, here, (keep >> s) & 1u, solid ? C(0) : d[s]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   auto plane_step = [&](int p, auto second) {
     first_step(f);
+    if constexpr (MASK) {  // c_z > 0 of plane p: what its blocked links send back
+#pragma unroll
+      for (int s = 0; s < Q; s++)
+        if (Lattice<Q>::c(s, 2) > 0 && blocked(lk, s)) next[s] = f[Lattice<Q>::opp(s)];
+    }
+    const uint32_t lk_after = load_links(p + 2);
     load_plane(p + 1, f);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();  // LDS holds plane p
@@ -211,17 +337,22 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
     for (int s = 0; s < Q; s++) {
       const int cz = Lattice<Q>::c(s, 2);
       if (cz == 0) {
-        h[s] = receive(s);
+        h[s] = receive(s, blocked(lk, s));
       } else if (cz > 0) {
         h[s] = next[s];
-        next[s] = receive(s);
+        next[s] = receive(s, false);
+      } else if (MASK) {
+        h[s] = receive(s, true);
       }
       // In registers before the barrier that lets the LDS be overwritten: the
       // compiler has moved such a read, used only later, below the barrier.
-      if (cz == 0) asm volatile("" : "+v"(h[s]));
+      if (cz == 0 || (MASK && cz < 0)) asm volatile("" : "+v"(h[s]));
       if (cz > 0) asm volatile("" : "+v"(h[s]), "+v"(next[s]));
     }
     __syncthreads();  // LDS has been read
+    lk_prev = lk;
+    lk = lk_next;
+    lk_next = lk_after;
   };
   plane_step(zc - 1, std::false_type{});
   plane_step(zc, std::false_type{});
@@ -237,58 +368,70 @@ struct PairKernel {
   size_t lds;
 };
 
-template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
 void launch_pair(hipStream_t stream, const void* f0, void* f1, const DenseArgs& a,
                  const PairArgs& pa) {
   using T = typename Storage<STORE>::T;
-  hipLaunchKernelGGL((k_dense_pair<Q, STORE, FORCE, NT, W, TY>), dim3(8 * pa.per_xcd),
+  hipLaunchKernelGGL((k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY>), dim3(8 * pa.per_xcd),
                      dim3(pair_threads<W, TY>()), (pair_lds_bytes<Q, STORE, W, TY>()), stream,
                      (const T*)f0, (T*)f1, a, pa);
 }
 
-template <int Q, int STORE, bool FORCE, bool NT, int W, int TY>
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
 PairKernel pair_kernel() {
-  return {launch_pair<Q, STORE, FORCE, NT, W, TY>,
-          (const void*)k_dense_pair<Q, STORE, FORCE, NT, W, TY>, W, TY, pair_threads<W, TY>(),
+  return {launch_pair<Q, STORE, MASK, FORCE, NT, W, TY>,
+          (const void*)k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY>, W, TY, pair_threads<W, TY>(),
           pair_lds_bytes<Q, STORE, W, TY>()};
 }
 
-template <int Q, int STORE, int W, int TY>
+template <int Q, int STORE, bool MASK, int W, int TY>
 PairKernel pick_pair_flags(bool force, bool nt) {
-  if (nt) return force ? pair_kernel<Q, STORE, true, true, W, TY>()
-                       : pair_kernel<Q, STORE, false, true, W, TY>();
-  return force ? pair_kernel<Q, STORE, true, false, W, TY>()
-               : pair_kernel<Q, STORE, false, false, W, TY>();
+  if (nt) return force ? pair_kernel<Q, STORE, MASK, true, true, W, TY>()
+                       : pair_kernel<Q, STORE, MASK, false, true, W, TY>();
+  return force ? pair_kernel<Q, STORE, MASK, true, false, W, TY>()
+               : pair_kernel<Q, STORE, MASK, false, false, W, TY>();
 }
 
 // Tile shapes: W = 64 cells of a row, or 32 for rows of up to 32 (a 24 x 200 x
 // 100 box, D3Q19 FP64: 18.4 us per step with 32 x 16 tiles, 24.1 with 64 x 8).
 // Large tiles have the smaller ring (512^3 D3Q19 FP64, 64 x 8: 4.10 ms per step,
-// 64 x 4: 5.03); the smaller ones give small boxes twice the workgroups.
-// D3Q27 FP64 spills registers in the 11-wave tiles and takes 64 x 4 and 32 x 8
-// always (384^3: 3.09 ms against 3.60).
-template <int Q, int STORE>
+// 64 x 4: 5.03); the smaller ones give small boxes twice the workgroups.  Waves
+// bound the registers: 11 of them (64 x 8) leave 168 per lane, which D3Q27 FP64
+// and masked D3Q19 FP64 exceed, and spills cost more than a larger ring (D3Q27
+// FP64 384^3: 64 x 4 3.09 ms, 64 x 8 3.60; masked channel with a force, 256^3
+// D3Q19 FP64: 64 x 5 778 us, 64 x 8 1,130).  Masked D3Q27 FP64 spills in every
+// tile and has no two-step kernel.
+template <int Q, int STORE, bool MASK>
 PairKernel pick_pair_tile(bool force, bool nt, bool narrow, bool small) {
-  if constexpr (!(Q == 27 && STORE == LBM_STORE_F64)) {
-    if (!small) return narrow ? pick_pair_flags<Q, STORE, 32, 16>(force, nt)
-                              : pick_pair_flags<Q, STORE, 64, 8>(force, nt);
+  if constexpr (MASK && STORE == LBM_STORE_F64) {
+    if constexpr (Q == 27) return {};
+    else return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 10>(force, nt)
+                       : pick_pair_flags<Q, STORE, MASK, 64, 5>(force, nt);
+  } else {
+    if constexpr (!(Q == 27 && STORE == LBM_STORE_F64)) {
+      if (!small) return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 16>(force, nt)
+                                : pick_pair_flags<Q, STORE, MASK, 64, 8>(force, nt);
+    }
+    return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 8>(force, nt)
+                  : pick_pair_flags<Q, STORE, MASK, 64, 4>(force, nt);
   }
-  return narrow ? pick_pair_flags<Q, STORE, 32, 8>(force, nt)
-                : pick_pair_flags<Q, STORE, 64, 4>(force, nt);
 }
 
-template <int Q>
+template <int Q, bool MASK>
 PairKernel pick_pair_q(int storage, bool force, bool nt, bool narrow, bool small) {
   switch (storage) {
-    case LBM_STORE_F64: return pick_pair_tile<Q, LBM_STORE_F64>(force, nt, narrow, small);
-    case LBM_STORE_F32S: return pick_pair_tile<Q, LBM_STORE_F32S>(force, nt, narrow, small);
+    case LBM_STORE_F64: return pick_pair_tile<Q, LBM_STORE_F64, MASK>(force, nt, narrow, small);
+    case LBM_STORE_F32S: return pick_pair_tile<Q, LBM_STORE_F32S, MASK>(force, nt, narrow, small);
   }
   return {};
 }
 
-// Defined in lbm_dense_pair19.hip and lbm_dense_pair27.hip; launch is nullptr
-// where there is no two-step kernel.  narrow: W = 32; small: half the rows.
+// Defined in lbm_dense_pair{19,27}.hip and, masked, lbm_dense_pair{19,27}_mask.hip;
+// launch is nullptr where there is no two-step kernel.  narrow: W = 32; small:
+// half the rows.
 PairKernel pick_pair19(int storage, bool force, bool nt, bool narrow, bool small);
 PairKernel pick_pair27(int storage, bool force, bool nt, bool narrow, bool small);
+PairKernel pick_pair19_mask(int storage, bool force, bool nt, bool narrow, bool small);
+PairKernel pick_pair27_mask(int storage, bool force, bool nt, bool narrow, bool small);
 
 }  // namespace lbm

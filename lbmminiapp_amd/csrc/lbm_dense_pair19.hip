@@ -3,6 +3,6 @@
 
 namespace lbm {
 PairKernel pick_pair19(int storage, bool force, bool nt, bool narrow, bool small) {
-  return pick_pair_q<19>(storage, force, nt, narrow, small);
+  return pick_pair_q<19, false>(storage, force, nt, narrow, small);
 }
 }  // namespace lbm

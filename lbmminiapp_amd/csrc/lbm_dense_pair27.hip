@@ -3,6 +3,6 @@
 
 namespace lbm {
 PairKernel pick_pair27(int storage, bool force, bool nt, bool narrow, bool small) {
-  return pick_pair_q<27>(storage, force, nt, narrow, small);
+  return pick_pair_q<27, false>(storage, force, nt, narrow, small);
 }
 }  // namespace lbm

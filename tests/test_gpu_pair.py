@@ -49,6 +49,44 @@ def test_pairs_equal_single_steps_f32(q, size, monkeypatch):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("periodic", [(1, 1, 1), (1, 0, 1), (0, 0, 0), (0, 1, 1), (1, 1, 0)],
+                         ids=lambda p: "".join(map(str, p)))
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_masked_pairs(size, periodic, monkeypatch):
+    """Walls and random solids, against the oracle (FP64) and single steps (FP32, pressure drop);
+    the state, the mass and the moments read back through walls."""
+    ncell = size[0] * size[1] * size[2]
+    solid = (O.uniform01(7, np.arange(ncell, dtype=np.uint64)) < 0.3).astype(np.uint8)
+    for mask in (None, solid):
+        if mask is None and periodic == (1, 1, 1):
+            continue
+        if mask is not None and mask.all():
+            continue
+        g = O.DenseGeometry(*size, mask, periodic=periodic)
+        fc = seeded_fc(g, 19)
+        full = np.zeros((19, ncell))
+        full[:, g.cell_of_fluid] = fc
+        for pattern, force in (("pull", (0.0, 0.0, 0.0)), ("aa", (1e-4, -2e-4, 3e-4))):
+            print(f"[pair] masked {size} {periodic} {mask is not None} {pattern}", flush=True)
+            got = run(monkeypatch, "1", size, full, 5, pattern="aa" if pattern == "aa" else "ab",
+                      pull=pattern == "pull", omega=1 / 0.6, force=force, solid=mask, periodic=periodic)
+            want = np.zeros_like(full)
+            want[:, g.cell_of_fluid] = oracle_run(g, 19, fc, pattern, 5, 1 / 0.6, force)
+            assert np.array_equal(got, want)
+        for q in (19, 27):
+            out = []
+            for pair in "01":
+                monkeypatch.setenv("LBM_DENSE_PAIR", pair)
+                with DenseLattice(*size, q=q, pattern="ab", pull=True, storage="f32s", omega=1 / 0.6,
+                                  solid=mask, periodic=periodic,
+                                  density_jump_x=3e-3 if periodic[0] else 0.0) as lat:
+                    lat.init_tgv(0.05, 1e-3, 3)
+                    lat.step(5)
+                    out.append((lat.get_state(), *lat.moments(), lat.mass()))
+            assert all(np.array_equal(a, b) for a, b in zip(out[0][:3], out[1][:3]))
+            assert abs(out[0][3] - out[1][3]) <= 1e-12 * out[0][3]
+
+
 def test_pairs_grouping_and_graphs(monkeypatch):
     """However the steps are grouped, and replayed from either array, the states are the same."""
     size, q = (70, 20, 9), 19
