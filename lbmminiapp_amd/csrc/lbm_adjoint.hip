@@ -638,9 +638,9 @@ lbm_status lbm_adjoint_backward(lbm_adjoint* h, double* grad_gamma, double* grad
   if (elapsed_ms) *elapsed_ms = ms;
   h->lam_cur = cur;
   if (grad_gamma)
-    LBM_HIP_CHECK(hipMemcpy(grad_gamma, h->grad[0], sizeof(double) * d->ncell, hipMemcpyDeviceToHost));
+    LBM_HIP_CHECK(copy_to_host(d->stage, d->stream, grad_gamma, h->grad[0], sizeof(double) * d->ncell));
   if (grad_tau)
-    LBM_HIP_CHECK(hipMemcpy(grad_tau, h->grad[1], sizeof(double) * d->ncell, hipMemcpyDeviceToHost));
+    LBM_HIP_CHECK(copy_to_host(d->stage, d->stream, grad_tau, h->grad[1], sizeof(double) * d->ncell));
   return LBM_OK;
 }
 
@@ -648,13 +648,10 @@ lbm_status lbm_adjoint_get_lambda0(lbm_adjoint* h, double* lam) {
   LBM_REQUIRE(h && lam, LBM_ERR_ARG, "lbm_adjoint_get_lambda0: null pointer");
   lbm_dense* d = h->d;
   const int64_t nq = d->ncell * d->q;
-  if (d->storage == LBM_STORE_F64) {
-    LBM_HIP_CHECK(hipMemcpy(lam, h->lam[h->lam_cur], sizeof(double) * nq, hipMemcpyDeviceToHost));
-  } else {
-    std::vector<float> tmp(nq);
-    LBM_HIP_CHECK(hipMemcpy(tmp.data(), h->lam[h->lam_cur], sizeof(float) * nq, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < nq; i++) lam[i] = tmp[i];
-  }
+  const bool f64 = d->storage == LBM_STORE_F64;
+  LBM_HIP_CHECK(copy_to_host(d->stage, d->stream, lam, h->lam[h->lam_cur],
+                             (f64 ? sizeof(double) : sizeof(float)) * nq,
+                             f64 ? HostCopy::PLAIN : HostCopy::F32_TO_F64));
   return LBM_OK;
 }
 

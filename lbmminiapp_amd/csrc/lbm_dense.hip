@@ -618,6 +618,7 @@ void free_all(lbm_dense* h) {
   if (h->omega_field) (void)hipFree(h->omega_field);
   if (h->gamma_field) (void)hipFree(h->gamma_field);
   if (h->partial) (void)hipFree(h->partial);
+  free_stage(h->stage);
   if (h->e0) (void)hipEventDestroy(h->e0);
   if (h->e1) (void)hipEventDestroy(h->e1);
   if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
@@ -1050,8 +1051,7 @@ lbm_status lbm_dense_get_state(lbm_dense* h, double* f) {
                                  h->stream, (const void*)h->f[h->cur], stage, h->args,
                                  canon_mode(h));
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(f, stage, bytes, hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) e = copy_to_host(h->stage, h->stream, f, stage, bytes);
   (void)hipFree(stage);
   if (e != hipSuccess) {
     set_error("lbm_dense_get_state: %s", hipGetErrorString(e));
@@ -1224,12 +1224,16 @@ lbm_status lbm_dense_moments(lbm_dense* h, double* rho, double* u) {
                            (const void*)h->f[h->cur], buf, buf + h->ncell, h->args,
                            canon_mode(h));
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(rho, buf, sizeof(double) * h->ncell, hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(u, buf + h->ncell, sizeof(double) * 3 * h->ncell, hipMemcpyDeviceToHost,
-                       h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  const size_t nb = sizeof(double) * h->ncell;
+  if (worth_staging(h->stage, 3 * nb)) {
+    if (e == hipSuccess) e = copy_to_host(h->stage, h->stream, u, buf + h->ncell, 3 * nb);
+    if (e == hipSuccess) e = copy_to_host(h->stage, h->stream, rho, buf, nb);
+  } else {
+    if (e == hipSuccess) e = hipMemcpyAsync(rho, buf, nb, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(u, buf + h->ncell, 3 * nb, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  }
   (void)hipFree(buf);
   if (e != hipSuccess) {
     set_error("lbm_dense_moments: %s", hipGetErrorString(e));

@@ -2,6 +2,7 @@
 // the adjoint module (lbm_adjoint.hip) shares with lbm_dense.hip.
 #pragma once
 #include "lbm_dense_pair.hpp"
+#include "lbm_host_copy.hpp"
 
 struct lbm_dense {
   int nx = 0, ny = 0, nz = 0, q = 19, pattern = 1, pull = 0, layout = 0, storage = 0;
@@ -38,6 +39,7 @@ struct lbm_dense {
   hipStream_t own_stream = nullptr;  // the handle's own stream (stream unless the caller set one)
   int live_graphs = 0;               // graphs captured from this handle and not yet destroyed
   hipEvent_t e0 = nullptr, e1 = nullptr;
+  lbm::HostStage stage;              // pinned staging of large readbacks
   lbm::DenseArgs args{};
   size_t device_bytes = 0;
 };
