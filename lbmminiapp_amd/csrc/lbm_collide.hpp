@@ -33,7 +33,7 @@ struct Dir {
 
 // sum of the non-zero terms c_d * a_d in d order (d = 0, 1, 2); 0 if none.
 template <typename T, int C0, int C1, int C2>
-__host__ __device__ inline T csum(T a0, T a1, T a2) {
+__host__ __device__ __forceinline__ T csum(T a0, T a1, T a2) {
   if constexpr (C0 == 0 && C1 == 0 && C2 == 0) {
     return T(0);
   } else {
@@ -57,7 +57,7 @@ __host__ __device__ inline T csum(T a0, T a1, T a2) {
 }
 
 template <int Q, typename T, int S>
-__host__ __device__ inline void moments_acc(const T* f, T& rho, T& v0, T& v1, T& v2) {
+__host__ __device__ __forceinline__ void moments_acc(const T* f, T& rho, T& v0, T& v1, T& v2) {
   rho += f[S];
   using D = Dir<Q, S>;
   if constexpr (D::cx > 0) v0 += f[S];
@@ -75,7 +75,7 @@ __host__ __device__ inline void moments_acc(const T* f, T& rho, T& v0, T& v1, T&
 // F = 0: 236 instead of 269 FP64 instructions per collision); every value is
 // rounded as the reference rounds it.
 template <int Q, typename T, int S, bool FORCE>
-__host__ __device__ inline void relax_ref(const T* f, T* out, T rho, T v0, T v1, T v2, T vdotv,
+__host__ __device__ __forceinline__ void relax_ref(const T* f, T* out, T rho, T v0, T v1, T v2, T vdotv,
                                           T fdotv, const T* F, double omega) {
 #pragma clang fp contract(off)
   using D = Dir<Q, S>;
@@ -116,7 +116,7 @@ __host__ __device__ inline void relax_ref(const T* f, T* out, T rho, T v0, T v1,
 // In-place or out-of-place: out may be f itself (each f[S] is read before out[S] is written).
 // FORCE = false requires F = (0, 0, 0) and then equals FORCE = true bit for bit.
 template <int Q, typename T, bool BRINKMAN, bool FORCE = true>
-__host__ __device__ inline void collide_ref(const T* f, T* out, double omega, const T* F,
+__host__ __device__ __forceinline__ void collide_ref(const T* f, T* out, double omega, const T* F,
                                             double gamma) {
 #pragma clang fp contract(off)
   T rho = 0.0;
@@ -144,7 +144,7 @@ __host__ __device__ inline void collide_ref(const T* f, T* out, double omega, co
 
 // ---------------------------------------------------------------- shifted storage
 template <int Q, int S>
-__host__ __device__ inline void moments_shift(const float* d, double& drho, double& m0, double& m1,
+__host__ __device__ __forceinline__ void moments_shift(const float* d, double& drho, double& m0, double& m1,
                                               double& m2) {
   const double x = (double)d[S];
   drho += x;
@@ -165,9 +165,9 @@ __host__ __device__ inline void moments_shift(const float* d, double& drho, doub
 //   even = om (drho + rho (cu^2/2 - uu/2)) + omf (cu cf - fu),  odd = om rho cu + omf cf
 // with uh = uu / 2, r = om rho and omd = om drho - omf fu.
 template <int Q, int S, bool FORCE>
-__host__ __device__ inline void relax_shift(float* d, float omd, float r, float a0, float a1,
+__host__ __device__ __forceinline__ void relax_shift(float* d, float omd, float r, float a0, float a1,
                                             float a2, float uh, float b0, float b1, float b2,
-                                            float keep, float omf) {
+                                            float keep) {
   using D = Dir<Q, S>;
   constexpr int O = Lattice<Q>::opp(S);
   constexpr float w = (float)Lattice<Q>::w(S);
@@ -176,25 +176,36 @@ __host__ __device__ inline void relax_shift(float* d, float omd, float r, float 
   } else if constexpr (S < O) {
     const float cu = csum<float, D::cx, D::cy, D::cz>(a0, a1, a2);
     float even = __builtin_fmaf(r, __builtin_fmaf(0.5f * cu, cu, -uh), omd);
-    float odd = r * cu;
+    float odd;
     if constexpr (FORCE) {
-      const float cf = omf * csum<float, D::cx, D::cy, D::cz>(b0, b1, b2);
+      const float cf = csum<float, D::cx, D::cy, D::cz>(b0, b1, b2);
       even = __builtin_fmaf(cu, cf, even);
-      odd += cf;
+      odd = __builtin_fmaf(r, cu, cf);
+    } else {
+      odd = r * cu;
     }
     d[S] = __builtin_fmaf(w, even + odd, keep * d[S]);
     d[O] = __builtin_fmaf(w, even - odd, keep * d[O]);
   }
   if constexpr (S + 1 < Q)
-    relax_shift<Q, S + 1, FORCE>(d, omd, r, a0, a1, a2, uh, b0, b1, b2, keep, omf);
+    relax_shift<Q, S + 1, FORCE>(d, omd, r, a0, a1, a2, uh, b0, b1, b2, keep);
 }
 
 // d[Q]: deviations f_s - w_s in FP32, updated in place.  FORCE = false requires F = 0.
-template <int Q, bool BRINKMAN, bool FORCE = true>
-__host__ __device__ inline void collide_shifted(float* d, double omega, const double* F,
-                                                double gamma) {
+// SCALED: d is scaled by `scale`, a power of two, and stays so; every rounding is
+// then the scaled one, and the results are the unscaled ones times `scale`.
+template <int Q, bool BRINKMAN, bool FORCE = true, bool SCALED = false>
+__host__ __device__ __forceinline__ void collide_shifted(float* d, double omega, const double* F,
+                                                double gamma, float scale = 1.0f,
+                                                float inv_scale = 1.0f) {
   double drho = 0.0, m0 = 0.0, m1 = 0.0, m2 = 0.0;
   moments_shift<Q, 0>(d, drho, m0, m1, m2);
+  if constexpr (SCALED) {
+    drho *= inv_scale;
+    m0 *= inv_scale;
+    m1 *= inv_scale;
+    m2 *= inv_scale;
+  }
   const double rho = 1.0 + drho;
   const double inv = 1.0 / rho;
   double u0 = (FORCE ? m0 + 0.5 * F[0] : m0) * inv;
@@ -205,19 +216,30 @@ __host__ __device__ inline void collide_shifted(float* d, double omega, const do
     u1 *= (1.0 - gamma);
     u2 *= (1.0 - gamma);
   }
-  const float fu0 = (float)u0, fu1 = (float)u1, fu2 = (float)u2;
+  // What all directions share is formed in FP64 and rounded once: a rounding that is
+  // common to them does not average out of the cell's mass and momentum.
   const float om = (float)omega, omf = 1.0f - 0.5f * om;
-  const float uh = 1.5f * __builtin_fmaf(fu2, fu2, __builtin_fmaf(fu1, fu1, fu0 * fu0));
-  float omd = om * (float)drho;
-  float F0 = 0.0f, F1 = 0.0f, F2 = 0.0f;  // 3 F
+  const float uh = (float)(1.5 * __builtin_fma(u2, u2, __builtin_fma(u1, u1, u0 * u0)));
+  double even = om * drho;
+  float F0 = 0.0f, F1 = 0.0f, F2 = 0.0f;  // 3 omf F
   if constexpr (FORCE) {
-    F0 = 3.0f * (float)F[0];
-    F1 = 3.0f * (float)F[1];
-    F2 = 3.0f * (float)F[2];
-    omd = __builtin_fmaf(-omf, __builtin_fmaf(F2, fu2, __builtin_fmaf(F1, fu1, F0 * fu0)), omd);
+    const double k = 3.0 * omf;
+    F0 = (float)(k * F[0]);
+    F1 = (float)(k * F[1]);
+    F2 = (float)(k * F[2]);
+    even = __builtin_fma(-k, __builtin_fma(F[2], u2, __builtin_fma(F[1], u1, F[0] * u0)), even);
   }
-  relax_shift<Q, 0, FORCE>(d, omd, om * (float)rho, 3.0f * fu0, 3.0f * fu1, 3.0f * fu2, uh, F0, F1,
-                           F2, 1.0f - om, omf);
+  float omd = (float)even;
+  float r = (float)(om * rho);
+  if constexpr (SCALED) {
+    omd *= scale;
+    r *= scale;
+    F0 *= scale;
+    F1 *= scale;
+    F2 *= scale;
+  }
+  relax_shift<Q, 0, FORCE>(d, omd, r, (float)(3.0 * u0), (float)(3.0 * u1), (float)(3.0 * u2), uh,
+                           F0, F1, F2, 1.0f - om);
 }
 
 }  // namespace lbm

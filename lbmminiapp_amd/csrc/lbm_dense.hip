@@ -26,7 +26,7 @@ enum CanonMode { C_LOCAL = 0, C_OPP = 1, C_GATHER = 2, C_WALL = 3 };
 // storage cell of cell = (x, y, z): on interleaved rows element x of the row
 // sits at position ir_pos(x)
 __device__ __forceinline__ int64_t store_cell(const DenseArgs& a, int64_t cell, int x) {
-  return a.xk ? cell - x + ir_pos(x, a.xk) : cell;
+  return a.xk ? cell - x + ir_pos(x, a.xk, a.xlg) : cell;
 }
 
 // storage index of f_s(x) for a given state convention
@@ -655,7 +655,7 @@ lbm_status init_from(lbm_dense* h, int src_kind, const double* rho_d, const doub
 // (64 planes: 545); 100^3 runs 12-plane chunks, 39.8 us (64 planes: 152).
 PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
   PairArgs p{};
-  p.ntx = (nx + k.w - 1) / k.w;
+  p.ntx = (nx / k.v + k.w - 1) / k.w;
   p.nty = (ny + k.ty - 1) / k.ty;
   double best = 0.0;
   for (int lz = 1; lz <= nz; lz++) {
@@ -671,8 +671,8 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
   return p;
 }
 
-// Two steps per launch (lbm_dense_pair.hpp) on SOA boxes in FP64 and FP32
-// deviations, without per-cell fields, and with a pressure drop only where there
+// Two steps per launch (lbm_dense_pair.hpp) on SOA boxes in FP64, FP32 and (even
+// unmasked rows) FP16 deviations, without per-cell fields, and with a pressure drop only where there
 // is a mask.  Default from 20,000 cells on; below, the march along z is a longer chain than two
 // launches (us per step, one step / two steps per launch, D3Q19 FP64: 16^3 3.9 /
 // 4.6, 128 x 16 x 8 3.8 / 5.4, 24^3 5.0 / 4.8, 28^3 6.3 / 5.0, 12 x 12 x 200
@@ -714,11 +714,34 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
       return 0;
     return cus * per_cu;
   };
-  const bool narrow = h->nx <= 32;
+  // cells per lane (split rows) and tile width, see lbm_dense_pair.hpp
+  auto lanes = [](int columns, int w) { return (columns + w - 1) / w * w; };
+  int v = 1;
+  if (h->storage == LBM_STORE_F16S) {
+    // no kernel with one cell per lane; small boxes and tiles that would be half
+    // empty keep single steps (us per step, single / pairs: 64^3 D3Q19 10.0 / 9.0,
+    // D3Q27 14.0 / 15.1, 32^3 4.3 / 5.8, 100^3 D3Q27 32.5 / 27.2; 320 x 100 x 90
+    // D3Q27, 17 % of the lanes empty, 59 / 61)
+    v = 2;
+    const int nc = h->nx / 2;
+    if (h->nx % 2 || need_links ||
+        (!e && (h->ncell < (h->q == 19 ? 250000 : 500000) ||
+                nc < (h->q == 19 ? 0.75 : 0.85) * lanes(nc, nc <= 32 ? 32 : 64))))
+      return;
+  } else if (h->storage == LBM_STORE_F32S && h->q == 19 && !need_links && h->nx % 2 == 0 &&
+             h->ncell >= ((int64_t)1 << 22) && 2 * lanes(h->nx / 2, 64) <= lanes(h->nx, 64)) {
+    v = 2;
+  }
+  if (const char* s = std::getenv("LBM_DENSE_PAIR_CELLS"))  // tuning: 1 or 2 where there is a choice
+    if (h->storage == LBM_STORE_F32S && h->q == 19 && !need_links && h->nx % 2 == 0)
+      v = std::atoi(s) == 2 ? 2 : 1;
+  const int nc = h->nx / v;
+  const bool narrow = nc <= 32 || (h->q == 19 && h->storage == LBM_STORE_F64 && !need_links &&
+                                   lanes(nc, 32) < 0.9 * lanes(nc, 64));
   // Small tiles where single planes of the large ones do not fill the GPU (32^3
   // D3Q19 FP64: 5.2 us per step against 6.7; 48^3, where they do: 9.6 / 8.7).
   for (const bool small : {false, true}) {
-    const PairKernel k = pick(h->storage, force, nt, narrow, small);
+    const PairKernel k = pick(h->storage, force, nt, narrow, small, v);
     const int s = k.launch ? slots(k) : 0;
     if (s <= 0) return;
     const PairArgs p = plan_pair(k, h->nx, h->ny, h->nz, s);
@@ -732,6 +755,8 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
     }
     h->pair = k;
     h->pair_args = p;
+    h->xk = v > 1 ? h->nx / v : 0;
+    h->xlg = v > 1 ? 1 : 6;
     if ((int64_t)p.ntx * p.nty * h->nz > s) return;
   }
 }
@@ -798,8 +823,10 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   if (aa_as_pairs) {
     size_t room = 0, total = 0;
     const size_t both = 2 * (size_t)h->ncell * h->q * h->esize;
-    if (hipMemGetInfo(&room, &total) != hipSuccess || both > total / 4 || both > room / 2)
+    if (hipMemGetInfo(&room, &total) != hipSuccess || both > total / 4 || both > room / 2) {
       h->pair = {};
+      h->xk = 0;
+    }
   }
   if (h->pair.launch) {
     h->pattern = LBM_PATTERN_AB;
@@ -823,6 +850,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
     const bool on = e ? e[0] != '0' : dflt;
     if (on && irows_ok && h->layout == LBM_LAYOUT_SOA && h->nx % 64 == 0) {
       h->xk = h->nx / 64;
+      h->xlg = 6;
       h->odd_seg_w = 0;
     }
   }
@@ -959,6 +987,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   a.inv_scale = (float)(1.0 / scale);
   a.djump = cfg->density_jump_x;
   a.xk = h->xk;
+  a.xlg = h->xlg;
   // With F = 0 the Guo terms are exact zeros, so the kernels that evaluate
   // them give the same bits as the specialised ones.  For D3Q19 FP64 AA on
   // SOA boxes without solids and with plain rows of more than 256 cells

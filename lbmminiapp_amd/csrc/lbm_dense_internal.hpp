@@ -19,7 +19,8 @@ struct lbm_dense {
   int slab_planes = 0;       // AA steps in pairs as z-slabs of this many planes (0: whole box)
   int odd_seg_w = 0;         // AA odd step as row segments of this width (k_dense_seg_odd; 0: off)
   size_t odd_seg_lds = 0;    // its dynamic LDS floor (caps workgroups per CU)
-  int xk = 0;                // interleaved rows: nx / 64 (0: plain rows)
+  int xk = 0;                // interleaved rows: nx / 64, split rows: nx / 2^xlg (0: plain rows)
+  int xlg = 6;
   int odd_ir_bx = 256;       // launch shape of the odd step on interleaved rows
   size_t odd_ir_lds = 0;
   lbm::PairKernel pair{};  // two time steps per launch (k_dense_pair); launch == nullptr: off

@@ -38,6 +38,16 @@
 // Work items go to the XCDs in contiguous runs (x fastest, then y, then chunks),
 // so that the tiles whose rings overlap share an L2.
 //
+// Split rows (V = 2): a lane takes the cells x and x + nx / 2, which are stored
+// side by side (ir_pos with blocks of two), so that its accesses are vectors of
+// two and a shift along x is one column for both; across the end of the row the
+// two parts change places.  It halves the instructions per byte: FP16 with one
+// cell per lane was no faster in pairs than in single steps (128-byte accesses),
+// with two 512^3 D3Q19 takes 1.34 ms per step (single steps 1.73), 128^3 25.5 us
+// (35.5).  FP32 D3Q19 gains from 4M cells on (512^3 2.59 -> 1.97 ms, 200 x 180 x
+// 220 0.210 -> 0.177; 100^3 20.0 -> 22.9 us); D3Q27 FP32 spills, and four cells per
+// lane were slower in FP16 (512^3 1.36 ms, 256^3 0.180 against 0.172).
+//
 // Masked boxes (MASK) hold their state through walls (K_AB_WALL): the gather
 // needs no links, so loads stay whole rows, and the stores put what a blocked
 // link sends back where the next gather looks for it.  Between the two steps a
@@ -48,12 +58,15 @@
 //
 // Measured, ms per step, one-step kernels -> pairs (tile as choose_pair takes it):
 //   D3Q19 FP64 512^3 7.15 -> 4.10   256^3 0.912 -> 0.493   128^3 0.110 -> 0.067
-//   D3Q19 FP32 512^3 3.42 -> 2.38   256^3 0.409 -> 0.266
+//   D3Q19 FP32 512^3 3.42 -> 1.97   256^3 0.409 -> 0.251
+//   D3Q19 FP16 512^3 1.73 -> 1.34   256^3 0.222 -> 0.172   D3Q27 FP16 256^3 0.324 -> 0.250
 //   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 384^3 2.40 -> 1.51
 //   channel with 5% spheres 256^3 D3Q19 FP64 0.930 -> 0.778   FP32 0.450 -> 0.338
 //   porous 384 x 250 x 260, 35% solid, D3Q19 FP64 1.37 -> 1.14   FP32 0.772 -> 0.618
 #pragma once
 #include "lbm_dense_kernels.hpp"
+
+#define LBM_INLINE __attribute__((always_inline))
 
 namespace lbm {
 
@@ -78,10 +91,30 @@ constexpr int pair_threads() {
   return W * TY + 2 * W + 64;
 }
 
-template <int Q, int STORE, int W, int TY>
+template <int Q, int STORE, int W, int TY, int V>
 constexpr size_t pair_lds_bytes() {
-  return (size_t)(Q - 3) * (W + 2) * (TY + 2) * sizeof(typename Storage<STORE>::C);
+  return (size_t)(Q - 3) * (W + 2) * (TY + 2) * V * sizeof(typename Storage<STORE>::T);
 }
+
+// V values of a lane: a vector, or for V = 1 the value itself.
+template <typename T, int V>
+struct Lanes {
+  typedef T type __attribute__((ext_vector_type(V)));
+  static __device__ __forceinline__ T get(type v, int i) { return v[i]; }
+  static __device__ __forceinline__ void set(type& v, int i, T x) { v[i] = x; }
+  // element i from i + d (mod V)
+  static __device__ __forceinline__ type turn(type v, int d) {
+    static_assert(V == 2, "two cells: either way is a swap");
+    return __builtin_shufflevector(v, v, 1, 0);
+  }
+};
+template <typename T>
+struct Lanes<T, 1> {
+  using type = T;
+  static __device__ __forceinline__ T get(T v, int) { return v; }
+  static __device__ __forceinline__ void set(T& v, int, T x) { v = x; }
+  static __device__ __forceinline__ T turn(T v, int) { return v; }
+};
 
 // A wave-uniform address kept in scalar registers, so that an access is one
 // instruction with a scalar base and the lane's 32-bit byte offset.
@@ -121,16 +154,19 @@ __device__ __forceinline__ void buffer_put(void* base, uint32_t bytes, uint32_t 
   }
 }
 
-template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY, int V>
 __global__ void __launch_bounds__((pair_threads<W, TY>()))
     k_dense_pair(const typename Storage<STORE>::T* __restrict__ f0,
                  typename Storage<STORE>::T* __restrict__ f1, DenseArgs a, PairArgs pa) {
   using T = typename Storage<STORE>::T;
   using C = typename Storage<STORE>::C;
-  static_assert(sizeof(T) == sizeof(C), "the first step's results are kept unrounded");
+  using L = Lanes<T, V>;
+  using VT = typename L::type;  // a lane's V cells: x, x + nc, x + 2 nc ... (split rows)
+  static_assert(V == 1 || !MASK, "masked boxes: plain rows");
   constexpr int EX = W + 2, EY = TY + 2, PL = EX * EY;
   extern __shared__ unsigned char lbm_smem[];
-  C* lds = reinterpret_cast<C*>(lbm_smem);  // [Q - 3][EY][EX]
+  VT* lds = reinterpret_cast<VT*>(lbm_smem);  // [Q - 3][EY][EX]
+  const int nc = a.nx / V;                    // columns of V cells
 
   int t = (blockIdx.x & 7) * pa.per_xcd + (blockIdx.x >> 3);
   if (t >= pa.ntx * pa.nty * pa.nch) return;
@@ -138,7 +174,7 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
   t /= pa.ntx;
   const int y0 = t % pa.nty * TY;
   const int zc = t / pa.nty * pa.lz, ze = zc + pa.lz < a.nz ? zc + pa.lz : a.nz;
-  const int xe = x0 + W < a.nx ? x0 + W : a.nx, ye = y0 + TY < a.ny ? y0 + TY : a.ny;
+  const int xe = x0 + W < nc ? x0 + W : nc, ye = y0 + TY < a.ny ? y0 + TY : a.ny;
 
   // The lane's cell (X, Y), which may lie one outside the box (the wrapped
   // neighbour); lanes past the end of the tile or of their role repeat a cell.
@@ -161,15 +197,15 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
     Y = Y < ye ? Y : ye;
   }
   const int lo = (Y - y0 + 1) * EX + X - x0 + 1;  // the cell's position in an LDS slot
-  const int x = wrap1(X, a.nx), y = wrap1(Y, a.ny);
+  const int x = wrap1(X, nc), y = wrap1(Y, a.ny);
   // byte offsets, within a plane, of the cells at (x - cx, y - cy)
   uint32_t off[3][3];
 #pragma unroll
   for (int i = 0; i < 3; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++)
-      off[i][j] = ((uint32_t)wrap1(y - (j - 1), a.ny) * (uint32_t)a.nx +
-                   (uint32_t)wrap1(x - (i - 1), a.nx)) * (uint32_t)sizeof(T);
+      off[i][j] = ((uint32_t)wrap1(y - (j - 1), a.ny) * (uint32_t)nc +
+                   (uint32_t)wrap1(x - (i - 1), nc)) * (uint32_t)sizeof(VT);
   const int64_t n = a.ncell, plane = (int64_t)a.nx * a.ny;
   const double F[3] = {a.F0, a.F1, a.F2};
 
@@ -182,22 +218,56 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
     return 0u;
   };
   // a population that crossed the periodic x boundary along an open link
-  auto jump = [&](C(&d)[Q], uint32_t k) {
-    if (MASK && a.djump != 0.0) {
+  auto jump = [&](VT(&d)[Q], uint32_t k) LBM_INLINE {
+    if constexpr (MASK) {
+      if (a.djump != 0.0) {
 #pragma unroll
-      for (int s = 0; s < Q; s++) {
-        const int cx = Lattice<Q>::c(s, 0);
-        const bool wall = (k >> Lattice<Q>::opp(s)) & 1u;
-        if (cx != 0) d[s] = with_jump<Q>(d[s], wall ? 0 : gather_crossing(cx, x, a.nx), s, a.djump);
+        for (int s = 0; s < Q; s++) {
+          const int cx = Lattice<Q>::c(s, 0);
+          const bool wall = (k >> Lattice<Q>::opp(s)) & 1u;
+          if (cx != 0) d[s] = with_jump<Q>(d[s], wall ? 0 : gather_crossing(cx, x, a.nx), s, a.djump);
+        }
       }
     }
   };
-  auto collide = [&](C* d) {
+  // the lane's cells, one after the other; FP16 deviations stay scaled
+  auto collide = [&](VT(&f)[Q]) LBM_INLINE {
     double G[3] = {F[0], F[1], F[2]};
     // masked FP64 keeps no products with the force in registers across the loop
     if constexpr (MASK && FORCE && STORE == LBM_STORE_F64)
       asm volatile("" : "+v"(G[0]), "+v"(G[1]), "+v"(G[2]));
-    collide_cell<Q, STORE, FORCE, false>(d, a.omega, G, nullptr, 0);
+    auto cell = [&](auto part) LBM_INLINE {
+      constexpr int i = decltype(part)::value;
+      C d[Q];
+#pragma unroll
+      for (int s = 0; s < Q; s++) d[s] = (C)L::get(f[s], i);
+      if constexpr (STORE == LBM_STORE_F64) collide_ref<Q, double, false, FORCE>(d, d, a.omega, G, 0.0);
+      else collide_shifted<Q, false, FORCE, STORE == LBM_STORE_F16S>(d, a.omega, G, 0.0, a.scale,
+                                                                     a.inv_scale);
+#pragma unroll
+      for (int s = 0; s < Q; s++) L::set(f[s], i, (T)d[s]);
+      if constexpr (V > 1) {
+        // packed again before the next part (the compiler would unpack all parts at once)
+        if constexpr (sizeof(VT) == 8) {
+#pragma unroll
+          for (int s = 0; s < Q; s++) {
+            uint64_t u = __builtin_bit_cast(uint64_t, f[s]);
+            asm volatile("" : "+v"(u));
+            f[s] = __builtin_bit_cast(VT, u);
+          }
+        } else if constexpr (sizeof(VT) == 4) {
+#pragma unroll
+          for (int s = 0; s < Q; s++) {
+            uint32_t u = __builtin_bit_cast(uint32_t, f[s]);
+            asm volatile("" : "+v"(u));
+            f[s] = __builtin_bit_cast(VT, u);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    cell(std::integral_constant<int, 0>{});
+    if constexpr (V > 1) cell(std::integral_constant<int, 1>{});
   };
   // ncell, opaque: the Q slot offsets are summed up again at each use rather than
   // kept in (and spilled from) scalar registers
@@ -206,7 +276,7 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)n));
   };
   // gathers the populations of plane p (past the chunk: of its last halo plane again)
-  auto load_plane = [&](int p, C(&f)[Q]) {
+  auto load_plane = [&](int p, VT(&f)[Q]) LBM_INLINE {
     const int z = wrap1(p < ze ? p : ze, a.nz);
     const T* src[3] = {f0 + plane * wrap1(z + 1, a.nz), f0 + plane * z,
                        f0 + plane * wrap1(z - 1, a.nz)};  // plane of cz = -1, 0, 1
@@ -216,14 +286,30 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
     for (int s = 0; s < Q; s++) {
       const auto base = scalar_base(src[Lattice<Q>::c(s, 2) + 1] + at);
       at += step;
-      f[s] = *(global_ptr<const T>)(
+      f[s] = *(global_ptr<const VT>)(
           base + lane_offset(off[Lattice<Q>::c(s, 0) + 1][Lattice<Q>::c(s, 1) + 1]));
     }
   };
-  C own[3];  // the first step's results that stay in the lane, by cz + 1
-  auto first_step = [&](C(&f)[Q]) {
+  VT own[3];  // the first step's results that stay in the lane, by cz + 1
+  auto first_step = [&](VT(&f)[Q], auto beside) LBM_INLINE {
+    if constexpr (V > 1) {
+      // across the end of the row, the neighbour of part i is in part i -+ 1
+#pragma unroll
+      for (int s = 0; s < Q; s++) {
+        const int cx = Lattice<Q>::c(s, 0);
+        if (cx > 0) f[s] = x == 0 ? L::turn(f[s], -1) : f[s];
+        if (cx < 0) f[s] = x == nc - 1 ? L::turn(f[s], 1) : f[s];
+      }
+    }
     jump(f, lk);
     collide(f);
+    if constexpr (V > 1 && decltype(beside)::value) {
+      // a wrapped column as the tile's end column sees it
+#pragma unroll
+      for (int s = 0; s < Q; s++)
+        if (pair_slot<Q>(s) >= 0)
+          f[s] = X < 0 ? L::turn(f[s], -1) : (X >= nc ? L::turn(f[s], 1) : f[s]);
+    }
 #pragma unroll
     for (int s = 0; s < Q; s++) {
       const int k = pair_slot<Q>(s);
@@ -233,13 +319,13 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  C f[Q];
+  VT f[Q];
   lk = load_links(zc - 1);
   lk_next = load_links(zc);
   load_plane(zc - 1, f);
   if (!inner) {
     for (int p = zc - 1; p <= ze; p++) {
-      first_step(f);
+      first_step(f, std::true_type{});
       const uint32_t lk_after = load_links(p + 2);
       load_plane(p + 1, f);
       __builtin_amdgcn_sched_barrier(0);
@@ -254,23 +340,23 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
   // Populations of the second step: h of cz = 0 and cz = 1 for plane p - 1, and
   // of cz = 1 for plane p (next), by direction.  Masked, h of cz = -1 is what a
   // blocked link sends back: the cell's own result in the opposite direction.
-  C h[Q] = {}, next[Q] = {};
+  VT h[Q] = {}, next[Q] = {};
   auto blocked = [&](uint32_t k, int s) { return MASK && ((k >> Lattice<Q>::opp(s)) & 1u); };
   // what the cell receives in direction s from the plane in LDS
-  auto receive = [&](int s, bool wall) -> C {
+  auto receive = [&](int s, bool wall) LBM_INLINE -> VT {
     const int k = pair_slot<Q>(s);
     if (k < 0) return own[(wall ? -1 : 1) * Lattice<Q>::c(s, 2) + 1];
     int pos = k * PL + lo - Lattice<Q>::c(s, 1) * EX - Lattice<Q>::c(s, 0);
     if (wall) pos = pair_slot<Q>(Lattice<Q>::opp(s)) * PL + lo;
     return lds[pos];
   };
-  auto second_step = [&](int z) {
-    C d[Q];
+  auto second_step = [&](int z) LBM_INLINE {
+    VT d[Q];
 #pragma unroll
     for (int s = 0; s < Q; s++) {
       d[s] = h[s];
       if (Lattice<Q>::c(s, 2) < 0) {
-        const C v = receive(s, false);
+        const VT v = receive(s, false);
         d[s] = blocked(lk_prev, s) ? h[s] : v;
       }
     }
@@ -282,7 +368,7 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
       const int64_t step = slot_stride();
 #pragma unroll
       for (int s = 0; s < Q; s++) {
-        const auto q = (global_ptr<T>)(scalar_base(dst) + lane_offset(here));
+        const auto q = (global_ptr<VT>)(scalar_base(dst) + lane_offset(here));
         dst += step;
         if constexpr (NT) __builtin_nontemporal_store(d[s], q);
         else *q = d[s];
@@ -308,21 +394,21 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
         const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
         if ((cx != 0 || cy != 0 || cz != 0) && ((wall >> s) & 1u)) {
           const auto base = scalar_base(f1 + (n * Lattice<Q>::opp(s) + plane * wrap1(z + cz, a.nz)));
-          *(global_ptr<T>)(base + lane_offset(off[1 - cx][1 - cy])) = d[s];
+          *(global_ptr<T>)(base + lane_offset(off[1 - cx][1 - cy])) = L::get(d[s], 0);
         }
       }
       T* dst = f1 + plane * z;
       const int64_t step = slot_stride();
 #pragma unroll
       for (int s = 0; s < Q; s++) {
-        buffer_put<NT>(dst + step * s, bytes, here, (keep >> s) & 1u, solid ? C(0) : d[s]);
+        buffer_put<NT>(dst + step * s, bytes, here, (keep >> s) & 1u, solid ? T(0) : L::get(d[s], 0));
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto plane_step = [&](int p, auto second) {
-    first_step(f);
+  auto plane_step = [&](int p, auto second) LBM_INLINE {
+    first_step(f, std::false_type{});
     if constexpr (MASK) {  // c_z > 0 of plane p: what its blocked links send back
 #pragma unroll
       for (int s = 0; s < Q; s++)
@@ -364,36 +450,38 @@ struct PairKernel {
   void (*launch)(hipStream_t stream, const void* f0, void* f1, const DenseArgs& a,
                  const PairArgs& pa);
   const void* fn;
-  int w, ty, threads;
+  int w, ty, v, threads;
   size_t lds;
 };
 
-template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY, int V>
 void launch_pair(hipStream_t stream, const void* f0, void* f1, const DenseArgs& a,
                  const PairArgs& pa) {
   using T = typename Storage<STORE>::T;
-  hipLaunchKernelGGL((k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY>), dim3(8 * pa.per_xcd),
-                     dim3(pair_threads<W, TY>()), (pair_lds_bytes<Q, STORE, W, TY>()), stream,
+  hipLaunchKernelGGL((k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY, V>), dim3(8 * pa.per_xcd),
+                     dim3(pair_threads<W, TY>()), (pair_lds_bytes<Q, STORE, W, TY, V>()), stream,
                      (const T*)f0, (T*)f1, a, pa);
 }
 
-template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY>
+template <int Q, int STORE, bool MASK, bool FORCE, bool NT, int W, int TY, int V>
 PairKernel pair_kernel() {
-  return {launch_pair<Q, STORE, MASK, FORCE, NT, W, TY>,
-          (const void*)k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY>, W, TY, pair_threads<W, TY>(),
-          pair_lds_bytes<Q, STORE, W, TY>()};
+  return {launch_pair<Q, STORE, MASK, FORCE, NT, W, TY, V>,
+          (const void*)k_dense_pair<Q, STORE, MASK, FORCE, NT, W, TY, V>, W, TY, V,
+          pair_threads<W, TY>(), pair_lds_bytes<Q, STORE, W, TY, V>()};
 }
 
-template <int Q, int STORE, bool MASK, int W, int TY>
+template <int Q, int STORE, bool MASK, int W, int TY, int V>
 PairKernel pick_pair_flags(bool force, bool nt) {
-  if (nt) return force ? pair_kernel<Q, STORE, MASK, true, true, W, TY>()
-                       : pair_kernel<Q, STORE, MASK, false, true, W, TY>();
-  return force ? pair_kernel<Q, STORE, MASK, true, false, W, TY>()
-               : pair_kernel<Q, STORE, MASK, false, false, W, TY>();
+  if (nt) return force ? pair_kernel<Q, STORE, MASK, true, true, W, TY, V>()
+                       : pair_kernel<Q, STORE, MASK, false, true, W, TY, V>();
+  return force ? pair_kernel<Q, STORE, MASK, true, false, W, TY, V>()
+               : pair_kernel<Q, STORE, MASK, false, false, W, TY, V>();
 }
 
-// Tile shapes: W = 64 cells of a row, or 32 for rows of up to 32 (a 24 x 200 x
-// 100 box, D3Q19 FP64: 18.4 us per step with 32 x 16 tiles, 24.1 with 64 x 8).
+// Tile shapes: W = 64 columns of a row, or 32 for rows of up to 32 (a 24 x 200 x
+// 100 box, D3Q19 FP64: 18.4 us per step with 32 x 16 tiles, 24.1 with 64 x 8) and,
+// D3Q19 FP64, where they leave a tenth fewer lanes empty (200 x 180 x 220: 269 us
+// against 287).
 // Large tiles have the smaller ring (512^3 D3Q19 FP64, 64 x 8: 4.10 ms per step,
 // 64 x 4: 5.03); the smaller ones give small boxes twice the workgroups.  Waves
 // bound the registers: 11 of them (64 x 8) leave 168 per lane, which D3Q27 FP64
@@ -401,37 +489,44 @@ PairKernel pick_pair_flags(bool force, bool nt) {
 // FP64 384^3: 64 x 4 3.09 ms, 64 x 8 3.60; masked channel with a force, 256^3
 // D3Q19 FP64: 64 x 5 778 us, 64 x 8 1,130).  Masked D3Q27 FP64 spills in every
 // tile and has no two-step kernel.
-template <int Q, int STORE, bool MASK>
+template <int Q, int STORE, bool MASK, int V>
 PairKernel pick_pair_tile(bool force, bool nt, bool narrow, bool small) {
   if constexpr (MASK && STORE == LBM_STORE_F64) {
     if constexpr (Q == 27) return {};
-    else return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 10>(force, nt)
-                       : pick_pair_flags<Q, STORE, MASK, 64, 5>(force, nt);
+    else return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 10, V>(force, nt)
+                       : pick_pair_flags<Q, STORE, MASK, 64, 5, V>(force, nt);
   } else {
     if constexpr (!(Q == 27 && STORE == LBM_STORE_F64)) {
-      if (!small) return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 16>(force, nt)
-                                : pick_pair_flags<Q, STORE, MASK, 64, 8>(force, nt);
+      if (!small) return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 16, V>(force, nt)
+                                : pick_pair_flags<Q, STORE, MASK, 64, 8, V>(force, nt);
     }
-    return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 8>(force, nt)
-                  : pick_pair_flags<Q, STORE, MASK, 64, 4>(force, nt);
+    return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 8, V>(force, nt)
+                  : pick_pair_flags<Q, STORE, MASK, 64, 4, V>(force, nt);
   }
 }
 
 template <int Q, bool MASK>
-PairKernel pick_pair_q(int storage, bool force, bool nt, bool narrow, bool small) {
-  switch (storage) {
-    case LBM_STORE_F64: return pick_pair_tile<Q, LBM_STORE_F64, MASK>(force, nt, narrow, small);
-    case LBM_STORE_F32S: return pick_pair_tile<Q, LBM_STORE_F32S, MASK>(force, nt, narrow, small);
+PairKernel pick_pair_q(int storage, bool force, bool nt, bool narrow, bool small, int v) {
+  if (storage == LBM_STORE_F64 && v == 1)
+    return pick_pair_tile<Q, LBM_STORE_F64, MASK, 1>(force, nt, narrow, small);
+  if (storage == LBM_STORE_F32S && v == 1)
+    return pick_pair_tile<Q, LBM_STORE_F32S, MASK, 1>(force, nt, narrow, small);
+  if constexpr (!MASK) {
+    if constexpr (Q == 19)
+      if (storage == LBM_STORE_F32S && v == 2)
+        return pick_pair_tile<Q, LBM_STORE_F32S, MASK, 2>(force, nt, narrow, small);
+    if (storage == LBM_STORE_F16S && v == 2)
+      return pick_pair_tile<Q, LBM_STORE_F16S, MASK, 2>(force, nt, narrow, small);
   }
   return {};
 }
 
 // Defined in lbm_dense_pair{19,27}.hip and, masked, lbm_dense_pair{19,27}_mask.hip;
 // launch is nullptr where there is no two-step kernel.  narrow: W = 32; small:
-// half the rows.
-PairKernel pick_pair19(int storage, bool force, bool nt, bool narrow, bool small);
-PairKernel pick_pair27(int storage, bool force, bool nt, bool narrow, bool small);
-PairKernel pick_pair19_mask(int storage, bool force, bool nt, bool narrow, bool small);
-PairKernel pick_pair27_mask(int storage, bool force, bool nt, bool narrow, bool small);
+// half the rows; v: cells per lane.
+PairKernel pick_pair19(int storage, bool force, bool nt, bool narrow, bool small, int v);
+PairKernel pick_pair27(int storage, bool force, bool nt, bool narrow, bool small, int v);
+PairKernel pick_pair19_mask(int storage, bool force, bool nt, bool narrow, bool small, int v);
+PairKernel pick_pair27_mask(int storage, bool force, bool nt, bool narrow, bool small, int v);
 
 }  // namespace lbm

@@ -2,7 +2,7 @@
 #include "lbm_dense_pair.hpp"
 
 namespace lbm {
-PairKernel pick_pair27_mask(int storage, bool force, bool nt, bool narrow, bool small) {
-  return pick_pair_q<27, true>(storage, force, nt, narrow, small);
+PairKernel pick_pair27_mask(int storage, bool force, bool nt, bool narrow, bool small, int v) {
+  return pick_pair_q<27, true>(storage, force, nt, narrow, small, v);
 }
 }  // namespace lbm
