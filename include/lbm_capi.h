@@ -175,7 +175,8 @@ typedef struct {
   int64_t n_fluid;           /* non-solid cells (MLUPS counts these) */
   int64_t time_step;         /* completed steps since the last set_state / init */
   double bytes_per_lup;      /* algorithmic HBM bytes per fluid-node update (2 Q b) */
-  size_t device_bytes;       /* device memory held by the handle */
+  size_t device_bytes;       /* device memory held by the handle (AA: one population array, or two
+                                where steps run in pairs and both fit a quarter of the device) */
 } lbm_dense_info;
 
 lbm_status lbm_dense_create(const lbm_dense_config* cfg, lbm_dense** out);
@@ -183,7 +184,7 @@ lbm_status lbm_dense_destroy(lbm_dense* h);
 lbm_status lbm_dense_get_info(lbm_dense* h, lbm_dense_info* info);
 /* Canonical pre-collision state in / out (host arrays of q * ncell doubles);
  * set_state resets time_step to 0.  Solid cells read back as 0.  The device
- * storage order (x-rows plain or interleaved, chosen at create) is internal:
+ * storage order (x-rows plain, interleaved or split, chosen at create) is internal:
  * every entry point takes and returns cell = x + nx * (y + ny * z) order. */
 lbm_status lbm_dense_set_state(lbm_dense* h, const double* f);
 lbm_status lbm_dense_get_state(lbm_dense* h, double* f);
