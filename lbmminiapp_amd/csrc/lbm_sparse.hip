@@ -510,7 +510,7 @@ lbm_status upload_adjacency(lbm_sparse* h, const int32_t* adjacency) {
   // 12.6 / 11.4, pull 12.6 / 11.5.  LBM_SPARSE_COMPRESS=0|1 overrides.
   const char* env = std::getenv("LBM_SPARSE_COMPRESS");
   const size_t esize = h->storage == LBM_STORE_F64 ? 8 : 4;
-  const bool compress = env ? env[0] != '0' : h->n * esize >= 1100000;
+  bool compress = env ? env[0] != '0' : h->n * esize >= 1100000;
   // one allocation: the caller's table, codes, tables of distances, raw flags
   const size_t words = h->q == 19 ? code_words<19>() : code_words<27>();
   auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -518,7 +518,13 @@ lbm_status upload_adjacency(lbm_sparse* h, const int32_t* adjacency) {
                code_b = pad(sizeof(uint32_t) * words * h->groups * kGroup),
                table_b = pad(sizeof(int32_t) * h->groups * h->q * kDeltas),
                raw_b = pad(sizeof(uint32_t) * h->groups);
-  if (hipMalloc(&h->adj, adj_b + (compress ? code_b + table_b + raw_b : 0)) != hipSuccess) {
+  // no room for the compressed form: the caller's table alone serves
+  if (compress && hipMalloc(&h->adj, adj_b + code_b + table_b + raw_b) != hipSuccess) {
+    (void)hipGetLastError();
+    h->adj = nullptr;
+    compress = false;
+  }
+  if (!compress && hipMalloc(&h->adj, adj_b) != hipSuccess) {
     h->adj = nullptr;
     set_error("lbm_sparse_create: hipMalloc of the adjacency failed");
     return LBM_ERR_OOM;
