@@ -143,15 +143,28 @@ __host__ __device__ __forceinline__ void collide_ref(const T* f, T* out, double 
 }
 
 // ---------------------------------------------------------------- shifted storage
-// FP64 moments of the deviations by direction pairs (S, opp(S)): their sum enters
-// the density, their difference the momentum (both exact but for deviations of
-// very different size).  The serial chain of the density is half as long as by
-// single directions: on a small grid, one wave per SIMD, a step is a latency
-// (13 x 137 x 16 channel D3Q19 FP16 10.2 -> 10.1 us); where arithmetic bounds,
-// D3Q19 FP16 pairs at 256^3 ran 3 % faster.
+// FP64 moments of the deviations, in slot order.
 template <int Q, int S>
 __host__ __device__ __forceinline__ void moments_shift(const float* d, double& drho, double& m0, double& m1,
                                               double& m2) {
+  const double x = (double)d[S];
+  drho += x;
+  using D = Dir<Q, S>;
+  if constexpr (D::cx > 0) m0 += x;
+  if constexpr (D::cx < 0) m0 -= x;
+  if constexpr (D::cy > 0) m1 += x;
+  if constexpr (D::cy < 0) m1 -= x;
+  if constexpr (D::cz > 0) m2 += x;
+  if constexpr (D::cz < 0) m2 -= x;
+  if constexpr (S + 1 < Q) moments_shift<Q, S + 1>(d, drho, m0, m1, m2);
+}
+
+// The same moments of FP16 values by direction pairs (S, opp(S)), with half the
+// serial chain: sums of FP16 values are exact in FP64 in any order (multiples of
+// 2^-24 below 2^22).
+template <int Q, int S>
+__host__ __device__ __forceinline__ void moments_f16(const float* d, double& drho, double& m0, double& m1,
+                                            double& m2) {
   using D = Dir<Q, S>;
   constexpr int O = Lattice<Q>::opp(S);
   if constexpr (S == O) {
@@ -166,56 +179,67 @@ __host__ __device__ __forceinline__ void moments_shift(const float* d, double& d
     if constexpr (D::cz > 0) m2 += diff;
     if constexpr (D::cz < 0) m2 -= diff;
   }
-  if constexpr (S + 1 < Q) moments_shift<Q, S + 1>(d, drho, m0, m1, m2);
+  if constexpr (S + 1 < Q) moments_f16<Q, S + 1>(d, drho, m0, m1, m2);
 }
 
-// Relaxation of the direction pairs (S, opp(S)) of the deviations.  The part of
-// the update that is even in c and the odd part are formed once per pair (D3Q19
-// at F = 0: 199 instead of 261 vector instructions per collision, moments included);
-// every FMA is written out, so that each kernel that collides rounds alike.
-//   even = om (drho + rho (cu^2/2 - uu/2)) + omf (cu cf - fu),  odd = om rho cu + omf cf
-// with uh = uu / 2, r = om rho and omd = om drho - omf fu.
+// Relaxation of the direction pairs (S, opp(S)) of the deviations.  Every FMA is
+// written out, so that each kernel that collides rounds alike:
+//   cu = 3 c.u, cf = 3 c.F, eqdev = drho + rho (cu + cu^2/2 - uu/2), fd = cf - fu + cu cf
+//   d = (1 - om) d + w (om eqdev + omf fd)
+// `force_fma`: which of the two products in brackets is the FMA's (FP16 deviations and
+// boxes with a Brinkman field: omf fd; otherwise om eqdev).  The opposite direction's cu and cf are the exact negatives, so a pair shares
+// them; every value is rounded as for single directions.
 template <int Q, int S, bool FORCE>
-__host__ __device__ __forceinline__ void relax_shift(float* d, float omd, float r, float a0, float a1,
-                                            float a2, float uh, float b0, float b1, float b2,
-                                            float keep) {
+__host__ __device__ __forceinline__ void relax_shift(float* d, float drho, float rho, float u0, float u1,
+                                            float u2, float uh, float fu, float F0, float F1,
+                                            float F2, float om, float omf, float keep,
+                                            bool force_fma) {
   using D = Dir<Q, S>;
   constexpr int O = Lattice<Q>::opp(S);
   constexpr float w = (float)Lattice<Q>::w(S);
+  auto relaxed = [&](float f, float e, float fd) {
+    const float eqdev = __builtin_fmaf(rho, e, drho);
+    float x = om * eqdev;
+    if constexpr (FORCE)
+      x = force_fma ? __builtin_fmaf(omf, fd, x) : __builtin_fmaf(om, eqdev, omf * fd);
+    return __builtin_fmaf(keep, f, w * x);
+  };
   if constexpr (D::cx == 0 && D::cy == 0 && D::cz == 0) {
-    d[S] = __builtin_fmaf(w, __builtin_fmaf(-r, uh, omd), keep * d[S]);
+    d[S] = relaxed(d[S], -uh, -fu);
   } else if constexpr (S < O) {
-    const float cu = csum<float, D::cx, D::cy, D::cz>(a0, a1, a2);
-    float even = __builtin_fmaf(r, __builtin_fmaf(0.5f * cu, cu, -uh), omd);
-    float odd;
+    const float cu = 3.0f * csum<float, D::cx, D::cy, D::cz>(u0, u1, u2);
+    const float hc = 0.5f * cu;
+    float fd = 0.0f, fdo = 0.0f;
     if constexpr (FORCE) {
-      const float cf = csum<float, D::cx, D::cy, D::cz>(b0, b1, b2);
-      even = __builtin_fmaf(cu, cf, even);
-      odd = __builtin_fmaf(r, cu, cf);
-    } else {
-      odd = r * cu;
+      const float sf = csum<float, D::cx, D::cy, D::cz>(F0, F1, F2), cf = 3.0f * sf;
+      fd = __builtin_fmaf(cu, cf, __builtin_fmaf(3.0f, sf, -fu));
+      fdo = __builtin_fmaf(cu, cf, __builtin_fmaf(-3.0f, sf, -fu));
     }
-    d[S] = __builtin_fmaf(w, even + odd, keep * d[S]);
-    d[O] = __builtin_fmaf(w, even - odd, keep * d[O]);
+    d[S] = relaxed(d[S], __builtin_fmaf(hc, cu, cu) - uh, fd);
+    d[O] = relaxed(d[O], __builtin_fmaf(hc, cu, -cu) - uh, fdo);
   }
   if constexpr (S + 1 < Q)
-    relax_shift<Q, S + 1, FORCE>(d, omd, r, a0, a1, a2, uh, b0, b1, b2, keep);
+    relax_shift<Q, S + 1, FORCE>(d, drho, rho, u0, u1, u2, uh, fu, F0, F1, F2, om, omf, keep,
+                                 force_fma);
 }
 
 // d[Q]: deviations f_s - w_s in FP32, updated in place.  FORCE = false requires F = 0.
-// SCALED: d is scaled by `scale`, a power of two, and stays so; every rounding is
-// then the scaled one, and the results are the unscaled ones times `scale`.
-template <int Q, bool BRINKMAN, bool FORCE = true, bool SCALED = false>
+// SCALED: d holds FP16 values as they are stored, scaled by `scale`, a power of two, and
+// stays scaled: every rounding is the scaled one, and the results are the unscaled ones
+// times `scale`.
+template <int Q, bool BRINKMAN, bool FORCE, bool SCALED = false>
 __host__ __device__ __forceinline__ void collide_shifted(float* d, double omega, const double* F,
-                                                double gamma, float scale = 1.0f,
+                                                double gamma, bool force_fma, float scale = 1.0f,
                                                 float inv_scale = 1.0f) {
   double drho = 0.0, m0 = 0.0, m1 = 0.0, m2 = 0.0;
-  moments_shift<Q, 0>(d, drho, m0, m1, m2);
   if constexpr (SCALED) {
+    moments_f16<Q, 0>(d, drho, m0, m1, m2);
     drho *= inv_scale;
     m0 *= inv_scale;
     m1 *= inv_scale;
     m2 *= inv_scale;
+  } else {
+    moments_shift<Q, 0>(d, drho, m0, m1, m2);
   }
   const double rho = 1.0 + drho;
   const double inv = 1.0 / rho;
@@ -227,30 +251,19 @@ __host__ __device__ __forceinline__ void collide_shifted(float* d, double omega,
     u1 *= (1.0 - gamma);
     u2 *= (1.0 - gamma);
   }
-  // What all directions share is formed in FP64 and rounded once: a rounding that is
-  // common to them does not average out of the cell's mass and momentum.
-  const float om = (float)omega, omf = 1.0f - 0.5f * om;
-  const float uh = (float)(1.5 * __builtin_fma(u2, u2, __builtin_fma(u1, u1, u0 * u0)));
-  double even = om * drho;
-  float F0 = 0.0f, F1 = 0.0f, F2 = 0.0f;  // 3 omf F
-  if constexpr (FORCE) {
-    const double k = 3.0 * omf;
-    F0 = (float)(k * F[0]);
-    F1 = (float)(k * F[1]);
-    F2 = (float)(k * F[2]);
-    even = __builtin_fma(-k, __builtin_fma(F[2], u2, __builtin_fma(F[1], u1, F[0] * u0)), even);
-  }
-  float omd = (float)even;
-  float r = (float)(om * rho);
+  const float fu0 = (float)u0, fu1 = (float)u1, fu2 = (float)u2;
+  const float F0 = (float)F[0], F1 = (float)F[1], F2 = (float)F[2];
+  const float uu = 3.0f * (fu0 * fu0 + fu1 * fu1 + fu2 * fu2);
+  const float fu = 3.0f * (F0 * fu0 + F1 * fu1 + F2 * fu2);
+  const float om = (float)omega;
+  float omf = 1.0f - 0.5f * om, sdrho = (float)drho, srho = (float)rho;
   if constexpr (SCALED) {
-    omd *= scale;
-    r *= scale;
-    F0 *= scale;
-    F1 *= scale;
-    F2 *= scale;
+    omf *= scale;
+    sdrho *= scale;
+    srho *= scale;
   }
-  relax_shift<Q, 0, FORCE>(d, omd, r, (float)(3.0 * u0), (float)(3.0 * u1), (float)(3.0 * u2), uh,
-                           F0, F1, F2, 1.0f - om);
+  relax_shift<Q, 0, FORCE>(d, sdrho, srho, fu0, fu1, fu2, 0.5f * uu, fu, F0, F1, F2, om, omf,
+                           1.0f - om, force_fma);
 }
 
 }  // namespace lbm

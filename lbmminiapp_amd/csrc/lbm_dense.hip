@@ -719,11 +719,15 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
   int v = 1;
   if (h->storage == LBM_STORE_F16S) {
     // no kernel with one cell per lane; small boxes and tiles that would be half
-    // empty keep single steps (us per step, single / pairs: 64^3 D3Q19 10.0 / 9.0,
-    // D3Q27 14.0 / 15.1, 32^3 4.3 / 5.8, 100^3 D3Q27 32.5 / 27.2; 320 x 100 x 90
-    // D3Q27, 17 % of the lanes empty, 59 / 61)
+    // empty keep single steps (us per step, single / pairs: 64^3 D3Q19 10.2 / 9.2,
+    // 32^3 4.5 / 6.3, 100^3 D3Q27 33.2 / 29.7; 320 x 100 x 90 D3Q27, 17 % of the
+    // lanes empty, 58 / 65)
+    // The kernel works on scaled values: the scale has to be a power of two.
     v = 2;
     const int nc = h->nx / 2;
+    int exponent = 0;
+    const double scale = cfg->f16_scale > 0.0 ? cfg->f16_scale : 4096.0;
+    if (std::frexp(scale, &exponent) != 0.5 || std::abs(exponent) > 32) return;
     if (h->nx % 2 || need_links ||
         (!e && (h->ncell < (h->q == 19 ? 250000 : 500000) ||
                 nc < (h->q == 19 ? 0.75 : 0.85) * lanes(nc, nc <= 32 ? 32 : 64))))

@@ -270,29 +270,21 @@ __device__ __forceinline__ bool leaves_box(const DenseArgs& a, int x, int y, int
 // same); otherwise separate bodies with and without the Brinkman term.  The
 // single body needs fewer VGPRs but schedules differently; which is faster
 // depends on the kernel (one_collision_body).
-// FP16 deviations stay scaled as they are stored (kAsStored: loads and stores of
-// the time-step kernels do not scale), which saves two products per population
-// and rounds each result once, to FP16.
-constexpr float kAsStored = 1.0f;
-template <int STORE>
-__device__ __forceinline__ double step_jump(const DenseArgs& a) {
-  return STORE == LBM_STORE_F16S ? a.djump * a.scale : a.djump;
-}
 template <int Q, int STORE, bool FORCE, bool ONE>
 __device__ __forceinline__ void collide_cell(typename Storage<STORE>::C* d, double om,
-                                             const double* F, const DenseArgs& a, int64_t cell) {
-  constexpr bool SCALED = STORE == LBM_STORE_F16S;
-  const double* gamma_field = a.gamma_field;
+                                             const double* F, const double* gamma_field,
+                                             int64_t cell) {
+  constexpr bool F16 = STORE == LBM_STORE_F16S;
   if constexpr (ONE) {
     const double gm = gamma_field ? gamma_field[cell] : 0.0;
     if constexpr (STORE == LBM_STORE_F64) collide_ref<Q, double, true, FORCE>(d, d, om, F, gm);
-    else collide_shifted<Q, true, FORCE, SCALED>(d, om, F, gm, a.scale, a.inv_scale);
+    else collide_shifted<Q, true, FORCE>(d, om, F, gm, F16 || gamma_field);
   } else if constexpr (STORE == LBM_STORE_F64) {
     if (gamma_field) collide_ref<Q, double, true, FORCE>(d, d, om, F, gamma_field[cell]);
     else collide_ref<Q, double, false, FORCE>(d, d, om, F, 0.0);
   } else {
-    if (gamma_field) collide_shifted<Q, true, FORCE, SCALED>(d, om, F, gamma_field[cell], a.scale, a.inv_scale);
-    else collide_shifted<Q, false, FORCE, SCALED>(d, om, F, 0.0, a.scale, a.inv_scale);
+    if (gamma_field) collide_shifted<Q, true, FORCE>(d, om, F, gamma_field[cell], true);
+    else collide_shifted<Q, false, FORCE>(d, om, F, 0.0, F16);
   }
 }
 
@@ -395,9 +387,9 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
           cross = gather_crossing(cx, xr, a.nx);
         }
         const auto* rp = row_of(f0, n, ss, a, yy, zz);
-        if (aligned) d[s] = ld_row<STORE, NT>(rp, (uint32_t)xx, kAsStored);
-        else d[s] = ld_row<STORE, false>(rp, (uint32_t)xx, kAsStored);
-        d[s] = with_jump<Q>(d[s], cross, s, step_jump<STORE>(a));
+        if (aligned) d[s] = ld_row<STORE, NT>(rp, (uint32_t)xx, a.inv_scale);
+        else d[s] = ld_row<STORE, false>(rp, (uint32_t)xx, a.inv_scale);
+        d[s] = with_jump<Q>(d[s], cross, s, a.djump);
         continue;
       }
       int64_t idx;
@@ -415,20 +407,20 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
           cross = bb ? 0 : gather_crossing(cx, xr, a.nx);
         }
       }
-      if (aligned && LAYOUT == LBM_LAYOUT_SOA) d[s] = ld_s<STORE, NT>(f0, idx, kAsStored);
-      else d[s] = ld<STORE>(f0, idx, kAsStored);
-      d[s] = with_jump<Q>(d[s], cross, s, step_jump<STORE>(a));
+      if (aligned && LAYOUT == LBM_LAYOUT_SOA) d[s] = ld_s<STORE, NT>(f0, idx, a.inv_scale);
+      else d[s] = ld<STORE>(f0, idx, a.inv_scale);
+      d[s] = with_jump<Q>(d[s], cross, s, a.djump);
     }
 
     const double om = a.omega_field ? a.omega_field[cell] : a.omega;
     const double F[3] = {a.F0, a.F1, a.F2};
-    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a, cell);
+    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a.gamma_field, cell);
   }
 
   if constexpr (ROWS) {
     auto put_row = [&](typename Storage<STORE>::T* rp, int xx, C v, bool aligned) {
-      if (aligned) st_row<STORE, NT>(rp, (uint32_t)xx, v, kAsStored);
-      else st_row<STORE, false>(rp, (uint32_t)xx, v, kAsStored);
+      if (aligned) st_row<STORE, NT>(rp, (uint32_t)xx, v, a.scale);
+      else st_row<STORE, false>(rp, (uint32_t)xx, v, a.scale);
     };
 #pragma unroll
     for (int s = 0; s < Q; s++) {
@@ -438,19 +430,19 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
         put_row(row_of(f1, n, s, a, y, z), x, d[s], true);
       } else if constexpr (IR) {
         put_row(row_of(f1, n, o, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)), ir_shift(x, cx, a.xk),
-                with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, step_jump<STORE>(a)), true);
+                with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, a.djump), true);
       } else {
         // streaming target: AA odd writes slot opp(s) at x + c_s, AB push slot s
         put_row(row_of(f1, n, KIND == K_AA_ODD ? o : s, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)),
                 permuted ? ir_shift(x, cx, a.xk, lg) : wrap1(x + cx, a.nx),
-                with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, step_jump<STORE>(a)), cx == 0 || irows);
+                with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, a.djump), cx == 0 || irows);
       }
     }
     return;
   }
   auto put = [&](int64_t idx, C v, bool aligned) {
-    if (aligned && LAYOUT == LBM_LAYOUT_SOA) st_s<STORE, NT>(f1, idx, v, kAsStored);
-    else st<STORE>(f1, idx, v, kAsStored);
+    if (aligned && LAYOUT == LBM_LAYOUT_SOA) st_s<STORE, NT>(f1, idx, v, a.scale);
+    else st<STORE>(f1, idx, v, a.scale);
   };
 #pragma unroll
   for (int s = 0; s < Q; s++) {
@@ -472,7 +464,7 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
       const int64_t sidx = slot<Q, LAYOUT>(n, KIND == K_AA_ODD ? o : s, cell + off.at(cx, cy, cz));
       const bool bb = MASK && ((lk >> s) & 1u);
       if (!bb) {
-        if (!solid) put(sidx, with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, step_jump<STORE>(a)), aligned);
+        if (!solid) put(sidx, with_jump<Q>(d[s], scatter_crossing(cx, xr, a.nx), s, a.djump), aligned);
       } else {
         // halfway bounce-back slot: AA odd slot s at x, AB push slot opp(s) at x
         const int64_t bidx = slot<Q, LAYOUT>(n, KIND == K_AA_ODD ? s : o, cell);
@@ -553,11 +545,11 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, kDenseMaxBlock),
       if constexpr (GATHER) {
         // element x of slot s in row (y - cy, z - cz)
         const C v = ld_row<STORE, NT>(
-            row_of(f0, n, s, a, wrap1(y - cy, a.ny), wrap1(z - cz, a.nz)), (uint32_t)x, kAsStored);
+            row_of(f0, n, s, a, wrap1(y - cy, a.ny), wrap1(z - cz, a.nz)), (uint32_t)x, a.inv_scale);
         if (cx == 0) d[s] = v;
         else lds[(k++) * nx + x] = v;
       } else {
-        d[s] = ld_row<STORE, NT>(row_of(f0, n, s, a, y, z), (uint32_t)x, kAsStored);
+        d[s] = ld_row<STORE, NT>(row_of(f0, n, s, a, y, z), (uint32_t)x, a.inv_scale);
       }
     }
   }
@@ -570,7 +562,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, kDenseMaxBlock),
       if (cx != 0) {
         int xs = x - cx;
         xs = xs < 0 ? xs + nx : (xs >= nx ? xs - nx : xs);
-        d[s] = with_jump<Q>(lds[(k++) * nx + xs], gather_crossing(cx, x, nx), s, step_jump<STORE>(a));
+        d[s] = with_jump<Q>(lds[(k++) * nx + xs], gather_crossing(cx, x, nx), s, a.djump);
       }
     }
   }
@@ -584,14 +576,14 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, kDenseMaxBlock),
     for (int s = 0; s < Q; s++) {
       const int o = Lattice<Q>::opp(s);
       if (!solid && ((lk >> o) & 1u))
-        d[s] = ld_row<STORE, NT>(row_of(f0, n, o, a, y, z), (uint32_t)x, kAsStored);
+        d[s] = ld_row<STORE, NT>(row_of(f0, n, o, a, y, z), (uint32_t)x, a.inv_scale);
     }
   }
 
   if (!solid) {
     const double om = a.omega_field ? a.omega_field[cell] : a.omega;
     const double F[3] = {a.F0, a.F1, a.F2};
-    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a, cell);
+    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a.gamma_field, cell);
   }
 
   if constexpr (SCATTER) {
@@ -604,11 +596,11 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, kDenseMaxBlock),
       const int tgt = KIND == K_AA_ODD ? o : s;
       if (cx == 0) {
         st_row<STORE, NT>(row_of(f1, n, tgt, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)),
-                          (uint32_t)x, d[s], kAsStored);
+                          (uint32_t)x, d[s], a.scale);
       } else {
         int xt = x + cx;
         xt = xt < 0 ? xt + nx : (xt >= nx ? xt - nx : xt);
-        lds[(k++) * nx + xt] = with_jump<Q>(d[s], scatter_crossing(cx, x, nx), s, step_jump<STORE>(a));
+        lds[(k++) * nx + xt] = with_jump<Q>(d[s], scatter_crossing(cx, x, nx), s, a.djump);
       }
     }
     __syncthreads();
@@ -620,13 +612,13 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(1, kDenseMaxBlock),
       const int tgt = KIND == K_AA_ODD ? o : s;
       if (cx != 0)
         st_row<STORE, NT>(row_of(f1, n, tgt, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)),
-                          (uint32_t)x, lds[(k++) * nx + x], kAsStored);
+                          (uint32_t)x, lds[(k++) * nx + x], a.scale);
     }
   } else {
     if (solid && !a.fill_solid) return;
 #pragma unroll
     for (int s = 0; s < Q; s++)
-      st_row<STORE, NT>(row_of(f1, n, s, a, y, z), (uint32_t)x, solid ? C(0) : d[s], kAsStored);
+      st_row<STORE, NT>(row_of(f1, n, s, a, y, z), (uint32_t)x, solid ? C(0) : d[s], a.scale);
   }
 }
 
@@ -710,7 +702,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
       }
     }
   }
-  const C hv = ld<STORE>(hp, 0, kAsStored);
+  const C hv = ld<STORE>(hp, 0, a.inv_scale);
   // keep the halo load ahead of the aligned ones: scheduled after them, its
   // latency would be waited out on its own before the first barrier
   __builtin_amdgcn_sched_barrier(0);
@@ -723,7 +715,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
       const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
       // element x of slot s in row (y - cy, z - cz)
       const T* rp = row_of(f, n, s, a, wrap1(y - cy, a.ny), wrap1(z - cz, a.nz));
-      const C val = ld_row<STORE, NT>(rp, (uint32_t)x, kAsStored);
+      const C val = ld_row<STORE, NT>(rp, (uint32_t)x, a.inv_scale);
       if (cx == 0) d[s] = val;
       else v[k++] = val;
     }
@@ -738,7 +730,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
     for (int s = 0; s < Q; s++) {
       const int cx = Lattice<Q>::c(s, 0);
       if (cx != 0) {
-        d[s] = with_jump<Q>(lds[k * L + 1 + tid - cx], gather_crossing(cx, x, nx), s, step_jump<STORE>(a));
+        d[s] = with_jump<Q>(lds[k * L + 1 + tid - cx], gather_crossing(cx, x, nx), s, a.djump);
         k++;
       }
     }
@@ -746,7 +738,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
   {
     const double om = a.omega_field ? a.omega_field[cell] : a.omega;
     const double F[3] = {a.F0, a.F1, a.F2};
-    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a, cell);
+    collide_cell<Q, STORE, FORCE, ONE>(d, om, F, a.gamma_field, cell);
   }
   __syncthreads();  // every LDS read of the gather is done
   {
@@ -757,9 +749,9 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
       const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
       if (cx == 0) {
         st_row<STORE, NT>(row_of(f, n, o, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)), (uint32_t)x,
-                          d[s], kAsStored);
+                          d[s], a.scale);
       } else {
-        lds[k * L + 1 + tid + cx] = with_jump<Q>(d[s], scatter_crossing(cx, x, nx), s, step_jump<STORE>(a));
+        lds[k * L + 1 + tid + cx] = with_jump<Q>(d[s], scatter_crossing(cx, x, nx), s, a.djump);
         k++;
       }
     }
@@ -779,7 +771,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
         T* rp = row_of(f, n, o, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz));
         // the element the neighbouring segment's node writes through its halo
         const bool foreign = (cx > 0 && tid == 0) || (cx < 0 && tid == W - 1);
-        if (!foreign) st_row<STORE, NT>(rp, (uint32_t)x, lds[k * L + 1 + tid], kAsStored);
+        if (!foreign) st_row<STORE, NT>(rp, (uint32_t)x, lds[k * L + 1 + tid], a.scale);
         if (tid == k) {
           sp = rp + (cx > 0 ? xr : xl);
           spos = k * L + (cx > 0 ? W + 1 : 0);
@@ -787,7 +779,7 @@ __global__ void __launch_bounds__(256) k_dense_seg_odd(typename Storage<STORE>::
         k++;
       }
     }
-    if (tid < NSH) st<STORE>(sp, 0, lds[spos], kAsStored);
+    if (tid < NSH) st<STORE>(sp, 0, lds[spos], a.scale);
   }
 }
 

@@ -43,10 +43,10 @@
 // two and a shift along x is one column for both; across the end of the row the
 // two parts change places.  It halves the instructions per byte: FP16 with one
 // cell per lane was no faster in pairs than in single steps (128-byte accesses),
-// with two 512^3 D3Q19 takes 1.34 ms per step (single steps 1.73), 128^3 25.5 us
-// (35.5).  FP32 D3Q19 gains from 4M cells on (512^3 2.59 -> 1.97 ms, 200 x 180 x
-// 220 0.210 -> 0.177; 100^3 20.0 -> 22.9 us); D3Q27 FP32 spills, and four cells per
-// lane were slower in FP16 (512^3 1.36 ms, 256^3 0.180 against 0.172).
+// with two 512^3 D3Q19 takes 1.45 ms per step (single steps 1.73), 128^3 27.5 us
+// (32.9).  FP32 D3Q19 gains from 4M cells on (512^3 2.57 -> 2.05 ms, 200 x 180 x
+// 220 0.209 -> 0.187; 160^3 79.0 -> 97.5 us); D3Q27 FP32 spills, and four cells per
+// lane were slower in FP16 (2% at 512^3, 5% at 256^3).
 //
 // Masked boxes (MASK) hold their state through walls (K_AB_WALL): the gather
 // needs no links, so loads stay whole rows, and the stores put what a blocked
@@ -54,15 +54,15 @@
 // blocked link takes the cell's own result instead of the neighbour's, from its
 // own LDS position or register.  Per-lane addresses chosen by link in the gather
 // made the pairs slower than single steps (384 x 250 x 260 porous, D3Q19 FP32:
-// 968 us per step; now 618, single steps 772).
+// 968 us per step; now 628, single steps 763).
 //
 // Measured, ms per step, one-step kernels -> pairs (tile as choose_pair takes it):
 //   D3Q19 FP64 512^3 7.15 -> 4.10   256^3 0.912 -> 0.493   128^3 0.110 -> 0.067
-//   D3Q19 FP32 512^3 3.42 -> 1.97   256^3 0.409 -> 0.251
-//   D3Q19 FP16 512^3 1.73 -> 1.34   256^3 0.222 -> 0.172   D3Q27 FP16 256^3 0.324 -> 0.250
-//   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 384^3 2.40 -> 1.51
-//   channel with 5% spheres 256^3 D3Q19 FP64 0.930 -> 0.778   FP32 0.450 -> 0.338
-//   porous 384 x 250 x 260, 35% solid, D3Q19 FP64 1.37 -> 1.14   FP32 0.772 -> 0.618
+//   D3Q19 FP32 512^3 3.39 -> 2.05   256^3 0.424 -> 0.268
+//   D3Q19 FP16 512^3 1.74 -> 1.45   256^3 0.219 -> 0.186   D3Q27 FP16 256^3 0.325 -> 0.263
+//   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 256^3 0.635 -> 0.414
+//   channel with 5% spheres 256^3 D3Q19 FP64 0.930 -> 0.778   FP32 0.456 -> 0.350
+//   porous 384 x 250 x 260, 35% solid, D3Q19 FP64 1.37 -> 1.14   FP32 0.763 -> 0.628
 #pragma once
 #include "lbm_dense_kernels.hpp"
 
@@ -230,6 +230,13 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
       }
     }
   };
+  // To the storage type.  FP16: the FP32 result is rounded first, as in the
+  // one-step kernels (one instruction for the last FMA and the conversion would
+  // round once).
+  auto pack = [&](C v) LBM_INLINE -> T {
+    if constexpr (STORE == LBM_STORE_F16S) asm("" : "+v"(v));
+    return (T)v;
+  };
   // the lane's cells, one after the other; FP16 deviations stay scaled
   auto collide = [&](VT(&f)[Q]) LBM_INLINE {
     double G[3] = {F[0], F[1], F[2]};
@@ -242,10 +249,10 @@ __global__ void __launch_bounds__((pair_threads<W, TY>()))
 #pragma unroll
       for (int s = 0; s < Q; s++) d[s] = (C)L::get(f[s], i);
       if constexpr (STORE == LBM_STORE_F64) collide_ref<Q, double, false, FORCE>(d, d, a.omega, G, 0.0);
-      else collide_shifted<Q, false, FORCE, STORE == LBM_STORE_F16S>(d, a.omega, G, 0.0, a.scale,
-                                                                     a.inv_scale);
+      else collide_shifted<Q, false, FORCE, STORE == LBM_STORE_F16S>(
+          d, a.omega, G, 0.0, STORE == LBM_STORE_F16S, a.scale, a.inv_scale);
 #pragma unroll
-      for (int s = 0; s < Q; s++) L::set(f[s], i, (T)d[s]);
+      for (int s = 0; s < Q; s++) L::set(f[s], i, pack(d[s]));
       if constexpr (V > 1) {
         // packed again before the next part (the compiler would unpack all parts at once)
         if constexpr (sizeof(VT) == 8) {
