@@ -577,10 +577,12 @@ bool caller_captures(const lbm_dense* h) {
 lbm_status enqueue_steps(lbm_dense* h, int nsteps) {
   int i = 0;
   if (h->pair.launch) {
-    // A caller's graph of an even run has to end in the array it starts in, as
-    // with one step per launch, so it records an even number of pairs.
+    // A caller's graph keeps the arrays it was captured with.  For a replay to find
+    // the state there, an even run has to end in the array it starts in, as with one
+    // step per launch: the captured run, and every run of the handle from then on.
+    if (caller_captures(h)) h->caller_graphs = true;
     int pairs = nsteps / 2;
-    if (pairs % 2 && caller_captures(h)) pairs--;
+    if (pairs % 2 && h->caller_graphs) pairs--;
     for (; i < 2 * pairs; i += 2) {
       h->pair.launch(h->stream, h->f[h->cur], h->f[1 - h->cur], h->args, h->pair_args);
       LBM_LAUNCH_CHECK();
@@ -637,13 +639,19 @@ lbm_status dmalloc(lbm_dense* h, void** p, size_t bytes, const char* what) {
   return LBM_OK;
 }
 
+// Step 0 again, in the array that an even step from here would be in: a caller's
+// graphs rely on it (enqueue_steps).  Without pairs of steps that is array 0.
+void restart(lbm_dense* h) {
+  h->cur = h->pair.launch ? h->cur ^ (int)(h->t & 1) : 0;
+  h->t = 0;
+}
+
 lbm_status init_from(lbm_dense* h, int src_kind, const double* rho_d, const double* u_d,
                      double u0, double noise, uint64_t seed) {
-  h->t = 0;
-  h->cur = 0;
+  restart(h);
   const int mode = canon_mode(h);
   launch_util<k_init_u>(h->q, h->storage, h->layout, grid_for(h), block_for(h->nx), h->stream,
-                        h->f[0], h->args, mode, src_kind, rho_d, u_d, u0, noise, seed);
+                        h->f[h->cur], h->args, mode, src_kind, rho_d, u_d, u0, noise, seed);
   LBM_LAUNCH_CHECK();
   return LBM_OK;
 }
@@ -1059,10 +1067,9 @@ lbm_status lbm_dense_set_state(lbm_dense* h, const double* f) {
   LBM_HIP_CHECK(hipMalloc(&stage, bytes));
   hipError_t e = hipMemcpyAsync(stage, f, bytes, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess) {
-    h->t = 0;
-    h->cur = 0;
+    restart(h);
     launch_util<k_set_canonical_u>(h->q, h->storage, h->layout, grid_for(h), block_for(h->nx),
-                                   h->stream, (const double*)stage, h->f[0], h->args,
+                                   h->stream, (const double*)stage, h->f[h->cur], h->args,
                                    canon_mode(h));
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
@@ -1241,7 +1248,12 @@ lbm_status lbm_dense_graph_launch(lbm_dense_graph* g, int32_t nlaunch) {
   LBM_REQUIRE((int)(h->t % 2) == g->phase && g->exec[h->cur], LBM_ERR_ARG,
               "lbm_dense_graph_launch: the handle is an odd number of steps away from the "
               "state the graph was captured in");
+  if (h->pair.launch && caller_captures(h)) h->caller_graphs = true;
   for (int32_t i = 0; i < nlaunch; i++) {
+    if (h->caller_graphs && g->end[h->cur] != h->cur) {  // see enqueue_steps
+      if (lbm_status st = enqueue_steps(h, g->nsteps)) return st;
+      continue;
+    }
     LBM_HIP_CHECK(hipGraphLaunch(g->exec[h->cur], h->stream));
     h->cur = g->end[h->cur];
     h->t += g->nsteps;

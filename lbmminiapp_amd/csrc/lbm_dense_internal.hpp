@@ -27,6 +27,7 @@ struct lbm_dense {
   lbm::PairArgs pair_args{};
   bool walls = false;        // state through walls (K_AB_WALL), masked boxes in pairs
   bool own_capture = false;  // lbm_dense_graph_create is recording
+  bool caller_graphs = false;  // a caller has recorded steps into a graph of its own
   int64_t ncell = 0, nfluid = 0, t = 0;
   size_t esize = 8;
   void* f[2] = {nullptr, nullptr};
