@@ -860,7 +860,8 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
     const bool dflt = h->pattern == LBM_PATTERN_AA && !need_links && h->nt &&
                       !(h->q == 27 && h->storage == LBM_STORE_F32S);
     const bool on = e ? e[0] != '0' : dflt;
-    if (on && irows_ok && h->layout == LBM_LAYOUT_SOA && h->nx % 64 == 0) {
+    // (the two-step kernels address plain or split rows)
+    if (on && irows_ok && !h->pair.launch && h->layout == LBM_LAYOUT_SOA && h->nx % 64 == 0) {
       h->xk = h->nx / 64;
       h->xlg = 6;
       h->odd_seg_w = 0;

@@ -1,0 +1,33 @@
+"""Two steps per launch asked for together with interleaved rows (LBM_DENSE_PAIR=1 and
+LBM_DENSE_IROWS=1): the states are those of single steps."""
+import numpy as np
+import pytest
+
+from lbmminiapp_amd.capi import DenseLattice
+from oracle import oracle as O
+from tests.test_gpu_dense import seeded_fc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32s", "f16s"])
+@pytest.mark.parametrize("masked", [False, True])
+def test_pairs_with_interleaved_rows_asked_for(storage, masked, monkeypatch):
+    size = (128, 11, 7)
+    n = size[0] * size[1] * size[2]
+    solid = (O.uniform01(7, np.arange(n, dtype=np.uint64)) < 0.3).astype(np.uint8) if masked else None
+    g = O.DenseGeometry(*size, solid)
+    f = np.zeros((19, n))
+    f[:, g.cell_of_fluid] = seeded_fc(g, 19)
+    out = []
+    for pair, irows in (("1", "1"), ("0", "0")):
+        monkeypatch.setenv("LBM_DENSE_PAIR", pair)
+        monkeypatch.setenv("LBM_DENSE_IROWS", irows)
+        monkeypatch.setenv("LBM_DENSE_PAIR_CELLS", "2")
+        print(f"[switches] {storage} masked={masked} pair={pair} irows={irows}", flush=True)
+        with DenseLattice(*size, storage=storage, solid=solid, omega=1 / 0.8) as lat:
+            lat.set_state(f)
+            lat.step(5)
+            out.append((lat.get_state(), *lat.moments(), lat.mass()))
+    assert all(np.array_equal(a, b) for a, b in zip(out[0][:3], out[1][:3]))
+    assert abs(out[0][3] - out[1][3]) <= 1e-12 * out[1][3]
