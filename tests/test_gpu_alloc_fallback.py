@@ -1,0 +1,61 @@
+"""The second population array of an AA box cannot be allocated (the device's memory ran out
+between the check and the allocation): lbm_dense_create goes on with one array, in place, and
+the handle's states are those of any other.  In a child process, where a small library in
+front of the HIP runtime asks it for far too much in place of that one allocation."""
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHIM = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+size_t fail_size = 0;  /* the second allocation of this size fails */
+int seen = 0;
+int hipMalloc(void** p, size_t n) {
+  static int (*real)(void**, size_t);
+  if (!real) real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+  if (n == fail_size && ++seen == 2) return real(p, (size_t)1 << 50);
+  return real(p, n);
+}
+"""
+
+CHILD = r"""
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+sys.path.insert(0, ".")
+import numpy as np
+from lbmminiapp_amd.capi import DenseLattice
+
+n = (64, 32, 24)
+one = 19 * 8 * n[0] * n[1] * n[2]
+out = []
+for fail in (0, one):
+    ctypes.c_size_t.in_dll(shim, "fail_size").value = fail
+    with DenseLattice(*n, omega=1 / 0.8) as lat:
+        left = ctypes.CDLL("libamdhip64.so.7").hipPeekAtLastError()
+        print("error left behind:", left, flush=True)
+        assert left == 0
+        print("[fallback]", fail, lat.info()["device_bytes"], flush=True)
+        assert (lat.info()["device_bytes"] < 2 * one) == bool(fail)
+        lat.init_tgv(0.05, 1e-4, 3)
+        lat.step(7)
+        out.append((lat.get_state(), *lat.moments()))
+assert ctypes.c_int.in_dll(shim, "seen").value >= 2
+assert all(np.array_equal(a, b) for a, b in zip(*out))
+print("same states")
+"""
+
+
+def test_create_in_place_after_failed_second_array(tmp_path):
+    (tmp_path / "shim.c").write_text(SHIM)
+    (tmp_path / "child.py").write_text(CHILD)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", tmp_path / "shim.so", tmp_path / "shim.c", "-ldl"],
+                   check=True)
+    r = subprocess.run([sys.executable, "-u", tmp_path / "child.py", tmp_path / "shim.so"],
+                       capture_output=True, text=True, timeout=100)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0 and "same states" in r.stdout
