@@ -196,7 +196,11 @@ lbm_status lbm_dense_init_equilibrium(lbm_dense* h, const double* rho, const dou
  * k = 2 pi / n per axis, plus noise * (2 U - 1) per component with
  * U = top53(splitmix64(seed * 0x9E3779B97F4A7C15 + 3 * cell + component)) / 2^53. */
 lbm_status lbm_dense_init_tgv(lbm_dense* h, double u0, double noise, uint64_t seed);
-/* Advance n steps (asynchronous).  PropagationAA::run / PropagationAB::run loop body. */
+/* Advance n steps (asynchronous).  PropagationAA::run / PropagationAB::run loop body.
+ * A handle that can take two steps per launch does so for calls of two and more; calls
+ * of one step in a row go back to single steps in the way of its pattern (AA: in place)
+ * where that is the faster one, at the third of them, and calls of more steps back into
+ * pairs, once 8 steps have been asked for.  A change costs about a step and a half. */
 lbm_status lbm_dense_step(lbm_dense* h, int32_t nsteps);
 /* Advance n steps and return their device time (HIP events on the handle's stream). */
 lbm_status lbm_dense_run_timed(lbm_dense* h, int32_t nsteps, double* elapsed_ms);

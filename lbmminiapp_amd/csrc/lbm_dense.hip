@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <utility>
 #include <vector>
 
 #include "lbm_dense_internal.hpp"
@@ -230,6 +231,24 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The state of every fluid cell from one gathering convention and row order into
+// another, in another array; values as they are stored.
+template <int Q, int STORE, int LAYOUT>
+__global__ void __launch_bounds__(256)
+    k_convert(const void* __restrict__ src, DenseArgs sa, int smode, void* __restrict__ dst,
+              DenseArgs da, int dmode) {
+  using T = typename Storage<STORE>::T;
+  int x, y, z;
+  int64_t cell;
+  if (!cell_coords(sa, x, y, z, cell)) return;
+  const uint32_t lk = sa.links ? sa.links[cell] : 0u;  // (masked boxes: plain rows)
+  if (lk & SOLID_BIT) return;
+  const Offsets off(x, y, z, sa.nx, sa.ny, sa.nz);
+  for (int s = 0; s < Q; s++)
+    static_cast<T*>(dst)[canon_index<Q, LAYOUT>(dmode, s, cell, x, lk, off, da)] =
+        static_cast<const T*>(src)[canon_index<Q, LAYOUT>(smode, s, cell, x, lk, off, sa)];
+}
+
 // ---------------------------------------------------------------- mass
 // Sum over every fluid cell of its Q stored values (any state convention but
 // through walls is a permutation of the canonical populations over the fluid
@@ -310,6 +329,7 @@ LBM_UTIL_KERNEL(k_get_canonical)
 LBM_UTIL_KERNEL(k_moments)
 LBM_UTIL_KERNEL(k_init)
 LBM_UTIL_KERNEL(k_mass_partial)
+LBM_UTIL_KERNEL(k_convert)
 #undef LBM_UTIL_KERNEL
 
 }  // namespace lbm
@@ -451,7 +471,7 @@ void set_launch_shapes(lbm_dense* h) {
 
 // state convention of the current array
 int canon_mode(const lbm_dense* h) {
-  if (h->pattern == LBM_PATTERN_AA) return (h->t % 2 == 0) ? C_OPP : C_GATHER;
+  if (h->pattern == LBM_PATTERN_AA) return h->opp ? C_OPP : C_GATHER;
   return h->walls ? C_WALL : (h->pull ? C_GATHER : C_LOCAL);
 }
 
@@ -550,7 +570,7 @@ lbm_status launch_kind(lbm_dense* h, int kind, void* f0, void* f1, int z0, int n
 // launches bit for bit.
 lbm_status enqueue_aa_pair_by_slabs(lbm_dense* h) {
   const int P = h->slab_planes, S = (h->nz + P - 1) / P;
-  void* f = h->f[0];
+  void* f = h->f[h->cur];
   auto run = [&](int kind, int k) {
     const int z0 = k * P;
     return launch_kind(h, kind, f, f, z0, std::min(P, h->nz - z0));
@@ -574,16 +594,76 @@ bool caller_captures(const lbm_dense* h) {
   return s == hipStreamCaptureStatusActive;
 }
 
+// The other way of storing the state and stepping, without moving the state.
+void swap_modes(lbm_dense* h) {
+  std::swap(static_cast<StepMode&>(*h), h->other);
+  h->in_pairs = !h->in_pairs;
+  h->args.xk = h->xk;
+  h->args.xlg = h->xlg;
+  h->ones = h->several = 0;
+}
+
+// ... with the state, which is in a gathering convention, into the other array.
+lbm_status convert_mode(lbm_dense* h) {
+  const DenseArgs from = h->args;
+  const int mode = canon_mode(h);
+  swap_modes(h);
+  h->opp = false;
+  launch_util<k_convert_u>(h->q, h->storage, h->layout, grid_for(h), block_for(h->nx), h->stream,
+                           (const void*)h->f[h->cur], from, mode, h->f[1 - h->cur], h->args,
+                           canon_mode(h));
+  LBM_LAUNCH_CHECK();
+  h->cur = 1 - h->cur;
+  return LBM_OK;
+}
+
+// One step of the present mode.
+lbm_status enqueue_step(lbm_dense* h) {
+  lbm_status st;
+  if (h->pattern == LBM_PATTERN_AA) {
+    st = launch_kind(h, h->opp ? K_AA_EVEN : K_AA_ODD, h->f[h->cur], h->f[h->cur]);
+    h->opp = !h->opp;
+  } else {
+    st = launch_kind(h, h->walls ? K_AB_WALL : (h->pull ? K_AB_PULL : K_AB_PUSH), h->f[h->cur],
+                     h->f[1 - h->cur]);
+    h->cur = 1 - h->cur;
+  }
+  h->t++;
+  return st;
+}
+
+// The mode for a call of `nsteps` steps; takes the first of them where the state has
+// to leave the AA even convention (whose stored values include the pressure jump)
+// before it can go into pairs.  A change of mode costs about a step and a half, so a
+// handle changes when the calls of a kind repeat: to pairs for 8 steps asked for in
+// calls of two and more, back at the third call of one step in a row.
+lbm_status choose_mode(lbm_dense* h, int nsteps, int* taken) {
+  h->ones = nsteps == 1 ? h->ones + 1 : 0;
+  h->several = nsteps == 1 ? 0 : std::min(h->several + nsteps, 8);
+  if (h->in_pairs) return h->alone_ok && h->ones >= 3 ? convert_mode(h) : LBM_OK;
+  if (h->alone_ok && h->several < 8) return LBM_OK;
+  if (h->pattern == LBM_PATTERN_AA && h->opp) {
+    if (lbm_status st = enqueue_step(h)) return st;
+    *taken = 1;
+  }
+  return convert_mode(h);
+}
+
 lbm_status enqueue_steps(lbm_dense* h, int nsteps) {
   int i = 0;
-  if (h->pair.launch) {
-    // A caller's graph keeps the arrays it was captured with.  For a replay to find
-    // the state there, an even run has to end in the array it starts in, as with one
-    // step per launch: the captured run, and every run of the handle from then on.
+  if (h->pair.launch && nsteps > 0) {
+    // A caller's graph keeps the arrays and the mode it was captured with.  For a
+    // replay to find the state there, an even run has to end in the array it starts
+    // in, as with one step per launch: the captured run, and every run of the handle
+    // from then on.
     if (caller_captures(h)) h->caller_graphs = true;
-    int pairs = nsteps / 2;
+    if (!h->caller_graphs && !h->own_capture)
+      if (lbm_status st = choose_mode(h, nsteps, &i)) return st;
+  }
+  if (h->in_pairs) {
+    int pairs = (nsteps - i) / 2;
     if (pairs % 2 && h->caller_graphs) pairs--;
-    for (; i < 2 * pairs; i += 2) {
+    for (; pairs > 0; pairs--, i += 2) {
       h->pair.launch(h->stream, h->f[h->cur], h->f[1 - h->cur], h->args, h->pair_args);
       LBM_LAUNCH_CHECK();
       h->cur = 1 - h->cur;
@@ -592,22 +672,14 @@ lbm_status enqueue_steps(lbm_dense* h, int nsteps) {
   }
   for (; i < nsteps; i++) {
     lbm_status st;
-    if (h->pattern == LBM_PATTERN_AA && h->slab_planes > 0 && h->t % 2 == 0 && i + 1 < nsteps) {
+    if (h->pattern == LBM_PATTERN_AA && h->slab_planes > 0 && h->opp && i + 1 < nsteps) {
       st = enqueue_aa_pair_by_slabs(h);
       if (st != LBM_OK) return st;
       h->t += 2;
       i++;
       continue;
     }
-    if (h->pattern == LBM_PATTERN_AA) {
-      st = launch_kind(h, (h->t % 2 == 0) ? K_AA_EVEN : K_AA_ODD, h->f[0], h->f[0]);
-    } else {
-      st = launch_kind(h, h->walls ? K_AB_WALL : (h->pull ? K_AB_PULL : K_AB_PUSH), h->f[h->cur],
-                       h->f[1 - h->cur]);
-      h->cur = 1 - h->cur;
-    }
-    if (st != LBM_OK) return st;
-    h->t++;
+    if ((st = enqueue_step(h)) != LBM_OK) return st;
   }
   return LBM_OK;
 }
@@ -641,8 +713,18 @@ lbm_status dmalloc(lbm_dense* h, void** p, size_t bytes, const char* what) {
 
 // Step 0 again, in the array that an even step from here would be in: a caller's
 // graphs rely on it (enqueue_steps).  Without pairs of steps that is array 0.
+// AA and push boxes with a pressure drop start in the mode without pairs: a
+// gathering convention would subtract the jump that its next step adds again, and
+// so round the state.
 void restart(lbm_dense* h) {
-  h->cur = h->pair.launch ? h->cur ^ (int)(h->t & 1) : 0;
+  if (!h->pair.launch) {
+    h->cur = 0;
+    h->opp = true;
+  } else {
+    if (h->starts_alone && h->in_pairs && !h->caller_graphs) swap_modes(h);
+    if (h->pattern == LBM_PATTERN_AB) h->cur ^= (int)(h->t & 1);
+    else h->opp = h->caller_graphs ? h->opp != (bool)(h->t & 1) : true;
+  }
   h->t = 0;
 }
 
@@ -685,8 +767,8 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
 // launches (us per step, one step / two steps per launch, D3Q19 FP64: 16^3 3.9 /
 // 4.6, 128 x 16 x 8 3.8 / 5.4, 24^3 5.0 / 4.8, 28^3 6.3 / 5.0, 12 x 12 x 200
 // 11.6 / 7.2; every larger size measured gained).  LBM_DENSE_PAIR=0|1 overrides;
-// a variable that tunes the one-step kernels asks for them.  Sets h->pair and
-// h->pair_args, and the cache policy: stores stream past the caches when both
+// a variable that tunes the one-step kernels asks for them.  Sets h->pair,
+// h->pair_args and the two-step mode, and the cache policy: stores stream past the caches when both
 // arrays exceed 320 MiB (100^3 FP64, 290 MiB: 44.0 us cached / 44.7 streaming;
 // 112^3, 408 MiB: 54.4 / 52.9; 120^3 FP32, 250 MiB: 34.4 / 39.8).
 // Masked boxes gain about 1.2x, so they take pairs only where the tiles waste
@@ -696,7 +778,8 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
 // reference's pipe, 20% of such rows, loses: simulationSize 2 12.5 / 14.4 us per
 // step, 4 59.5 / 74.7.  An AA box whose array fits the memory-side cache where
 // two do not keeps its one array (100^3 porous D3Q19 FP64 52.8 / 55.8).
-void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, double live) {
+void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, double live,
+                 StepMode* mode) {
   const char* e = std::getenv("LBM_DENSE_PAIR");
   bool on = h->ncell >= 20000;
   for (const char* v : {"LBM_DENSE_IROWS", "LBM_DENSE_ODD_SEG", "LBM_DENSE_SLAB_PLANES",
@@ -767,8 +850,12 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
     }
     h->pair = k;
     h->pair_args = p;
-    h->xk = v > 1 ? h->nx / v : 0;
-    h->xlg = v > 1 ? 1 : 6;
+    mode->pattern = LBM_PATTERN_AB;
+    mode->pull = 1;
+    mode->walls = need_links;
+    mode->nt = h->nt;
+    mode->xk = v > 1 ? h->nx / v : 0;
+    mode->xlg = v > 1 ? 1 : 6;
     if ((int64_t)p.ntx * p.nty * h->nz > s) return;
   }
 }
@@ -830,20 +917,15 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   // box they take a second population array, so only while both fit easily: a
   // quarter of the GPU's memory, and half of what is free (512^3 D3Q19 FP64:
   // 41 of 288 GB).  Larger boxes, and a GPU that is nearly full, step in place.
-  if (pair_ok) choose_pair(h, cfg, need_links, live);
+  StepMode paired;
+  if (pair_ok) choose_pair(h, cfg, need_links, live, &paired);
+  const size_t one_array = (size_t)h->ncell * h->q * h->esize;
   const bool aa_as_pairs = h->pair.launch && h->pattern == LBM_PATTERN_AA;
   if (aa_as_pairs) {
     size_t room = 0, total = 0;
-    const size_t both = 2 * (size_t)h->ncell * h->q * h->esize;
-    if (hipMemGetInfo(&room, &total) != hipSuccess || both > total / 4 || both > room / 2) {
+    if (hipMemGetInfo(&room, &total) != hipSuccess || 2 * one_array > total / 4 ||
+        2 * one_array > room / 2)
       h->pair = {};
-      h->xk = 0;
-    }
-  }
-  if (h->pair.launch) {
-    h->pattern = LBM_PATTERN_AB;
-    h->pull = 1;
-    h->walls = need_links;
   }
   // Interleaved rows (lbm_dense_kernels.hpp) for AA on unmasked periodic SOA
   // boxes whose rows are whole 64-element blocks: the odd step then makes only
@@ -860,8 +942,8 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
     const bool dflt = h->pattern == LBM_PATTERN_AA && !need_links && h->nt &&
                       !(h->q == 27 && h->storage == LBM_STORE_F32S);
     const bool on = e ? e[0] != '0' : dflt;
-    // (the two-step kernels address plain or split rows)
-    if (on && irows_ok && !h->pair.launch && h->layout == LBM_LAYOUT_SOA && h->nx % 64 == 0) {
+    // (a mask is stored once, and the two-step kernels address plain rows)
+    if (on && irows_ok && !(h->pair.launch && need_links) && h->layout == LBM_LAYOUT_SOA && h->nx % 64 == 0) {
       h->xk = h->nx / 64;
       h->xlg = 6;
       h->odd_seg_w = 0;
@@ -904,7 +986,7 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   }
   h->stream = h->own_stream;
   const size_t fbytes = (size_t)h->ncell * h->q * h->esize;
-  const int narrays = h->pattern == LBM_PATTERN_AA ? 1 : 2;
+  const int narrays = h->pattern == LBM_PATTERN_AA && !h->pair.launch ? 1 : 2;
   for (int i = 0; i < narrays; i++)
     if ((st = dmalloc(h, &h->f[i], fbytes, "populations"))) {
       (void)fail(st);
@@ -999,8 +1081,6 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   a.scale = (float)scale;
   a.inv_scale = (float)(1.0 / scale);
   a.djump = cfg->density_jump_x;
-  a.xk = h->xk;
-  a.xlg = h->xlg;
   // With F = 0 the Guo terms are exact zeros, so the kernels that evaluate
   // them give the same bits as the specialised ones.  For D3Q19 FP64 AA on
   // SOA boxes without solids and with plain rows of more than 256 cells
@@ -1017,10 +1097,33 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
     const char* e = std::getenv("LBM_DENSE_FORCE_TERMS");
     h->force_terms = e ? e[0] == '1' : dflt;
   }
+  // What has been set up so far is the mode without pairs.  Single steps go back to
+  // it where it is faster than out of place (us per step, in place / out of place,
+  // D3Q19): AA boxes whose two arrays exceed the memory-side cache (FP64 100^3 52.5 /
+  // 60.7, 512^3 7,090 / 7,880; FP32 128^3 46.9 / 59.5; below, FP64 64^3 15.8 / 13.4,
+  // FP32 100^3 31.5 / 29.3) or, masked, very small ones (32^3 FP32 5.8 / 6.4, 64^3
+  // 12.8 / 12.0); gathers through walls (pull / through walls: 64^3 channel FP32 8.8 /
+  // 12.0, porous 384 x 250 x 260 FP32 768 / 1,011) and split rows (pull, 64^3 FP16 7.9
+  // / 8.4), where it is the pull.
+  if (h->pair.launch) {
+    const bool aa = h->pattern == LBM_PATTERN_AA;
+    h->alone_ok = aa ? 2 * one_array > ((size_t)256 << 20) || (need_links && h->ncell < 40000)
+                     : (paired.walls && h->pull) || paired.xk;
+    h->starts_alone = a.djump != 0.0 && !(h->pattern == LBM_PATTERN_AB && h->pull);
+    if (!aa) {
+      // push: the state of the mode without pairs is one that pairs can take
+      if (h->starts_alone) h->pattern = LBM_PATTERN_AA;
+      h->pull = h->pattern == LBM_PATTERN_AB;
+    }
+    h->other = paired;
+    swap_modes(h);
+  }
+  a.xk = h->xk;
+  a.xlg = h->xlg;
   // rest state, as PropagationAA/AB::initialize (src/propagation/PropagationAA.cpp:60-123)
   if ((st = init_from(h, 0, nullptr, nullptr, 0.0, 0.0, 0))) return fail(st);
   // (the two-step kernels store every cell of the second array before it is read)
-  if (h->pattern == LBM_PATTERN_AB && !h->pair.launch &&
+  if (narrays == 2 && !h->pair.launch &&
       hipMemcpyAsync(h->f[1], h->f[0], fbytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) {
     set_error("lbm_dense_create: initial copy failed");
     return fail(LBM_ERR_HIP);
@@ -1166,9 +1269,10 @@ lbm_status lbm_dense_set_stream(lbm_dense* h, void* stream) {
 // brings an even run back to the array it started in, but two steps per launch
 // may not, and the handle may have changed arrays since the capture, so a
 // handle with two-step launches captures the run once from each array and
-// replays the one that starts in the current array.  The kernels take the
-// handle's device pointers, which stay fixed for the handle's lifetime; capture
-// records kernel launches only.
+// replays the one that starts in the current array; while it is in its mode
+// without pairs, a launch runs the steps as lbm_dense_step does.  The kernels take
+// the handle's device pointers, which stay fixed for the handle's lifetime;
+// capture records kernel launches only.
 struct lbm_dense_graph {
   lbm_dense* h = nullptr;
   int32_t nsteps = 0;
@@ -1176,6 +1280,7 @@ struct lbm_dense_graph {
   hipGraph_t graph[2] = {nullptr, nullptr};  // by the array the run starts in
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   int end[2] = {0, 0};                       // the array it ends in
+  bool pairs = false;                        // captured in the two-step mode
   bool counted = false;                      // included in h->live_graphs
 };
 
@@ -1211,11 +1316,16 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
   const hipStream_t user = h->stream;
   const int64_t t0 = h->t;
   const int cur0 = h->cur;
+  const bool opp0 = h->opp, in_pairs0 = h->in_pairs;
+  const int ones0 = h->ones, several0 = h->several;
   h->stream = cap;
   h->own_capture = true;
+  // (a handle whose mode a caller's graph holds on to is captured in that mode)
+  g->pairs = h->pair.launch && (h->in_pairs || !h->caller_graphs);
+  if (g->pairs != h->in_pairs) swap_modes(h);
   lbm_status st = LBM_OK;
   for (int c = 0; c < 2 && st == LBM_OK && e == hipSuccess; c++) {
-    if (!h->pair.launch && c != cur0) continue;
+    if (!g->pairs && c != cur0) continue;
     h->t = t0;
     h->cur = c;
     e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
@@ -1229,8 +1339,12 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
   }
   h->stream = user;
   h->own_capture = false;
+  if (in_pairs0 != h->in_pairs) swap_modes(h);
   h->t = t0;
   h->cur = cur0;
+  h->opp = opp0;
+  h->ones = ones0;
+  h->several = several0;
   (void)hipStreamDestroy(cap);
   if (st != LBM_OK || e != hipSuccess) {
     if (st == LBM_OK) set_error("lbm_dense_graph_create: %s", hipGetErrorString(e));
@@ -1246,15 +1360,17 @@ lbm_status lbm_dense_graph_create(lbm_dense* h, int32_t nsteps, lbm_dense_graph*
 lbm_status lbm_dense_graph_launch(lbm_dense_graph* g, int32_t nlaunch) {
   LBM_REQUIRE(g && nlaunch >= 0, LBM_ERR_ARG, "lbm_dense_graph_launch: bad arguments");
   lbm_dense* h = g->h;
-  LBM_REQUIRE((int)(h->t % 2) == g->phase && g->exec[h->cur], LBM_ERR_ARG,
+  if (h->pair.launch && caller_captures(h)) h->caller_graphs = true;
+  LBM_REQUIRE((int)(h->t % 2) == g->phase && (g->pairs || g->exec[h->cur]), LBM_ERR_ARG,
               "lbm_dense_graph_launch: the handle is an odd number of steps away from the "
               "state the graph was captured in");
-  if (h->pair.launch && caller_captures(h)) h->caller_graphs = true;
   for (int32_t i = 0; i < nlaunch; i++) {
-    if (h->caller_graphs && g->end[h->cur] != h->cur) {  // see enqueue_steps
+    // not the captured mode, or a caller's graph relies on the array (enqueue_steps)
+    if (g->pairs != h->in_pairs || (h->caller_graphs && g->end[h->cur] != h->cur)) {
       if (lbm_status st = enqueue_steps(h, g->nsteps)) return st;
       continue;
     }
+    h->ones = 0;
     LBM_HIP_CHECK(hipGraphLaunch(g->exec[h->cur], h->stream));
     h->cur = g->end[h->cur];
     h->t += g->nsteps;

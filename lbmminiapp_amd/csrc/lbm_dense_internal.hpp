@@ -4,8 +4,25 @@
 #include "lbm_dense_pair.hpp"
 #include "lbm_host_copy.hpp"
 
-struct lbm_dense {
-  int nx = 0, ny = 0, nz = 0, q = 19, pattern = 1, pull = 0, layout = 0, storage = 0;
+namespace lbm {
+
+// How a handle stores its state and takes single steps.  A handle with two-step
+// launches has two ways: in pairs (out of place, AB pull convention or through
+// walls, plain or split rows) and alone, the way a box without pairs steps.
+struct StepMode {
+  int pattern = 1, pull = 0;
+  bool walls = false;        // state through walls (K_AB_WALL)
+  bool nt = true;            // streaming (non-temporal) accesses in the time-step kernels
+  bool force_terms = false;  // time-step kernels with the Guo terms also at F = 0
+  int odd_seg_w = 0;         // AA odd step as row segments of this width (k_dense_seg_odd; 0: off)
+  int xk = 0;                // interleaved rows: nx / 64, split rows: nx / 2 (0: plain rows)
+  int xlg = 6;               // log2 of the row block: 6, split rows 1
+};
+
+}  // namespace lbm
+
+struct lbm_dense : lbm::StepMode {
+  int nx = 0, ny = 0, nz = 0, q = 19, layout = 0, storage = 0;
   int periodic[3] = {1, 1, 1};
   int staged_mode = 1;  // LDS-staged kernels: 0 never, 1 default cases, 2 every case they cover
   // launch shape of the unstaged time-step kernels (block width, dynamic LDS
@@ -14,20 +31,20 @@ struct lbm_dense {
   int step_bx = 256, even_bx = 256;
   size_t step_lds = 0, even_lds = 0;
   size_t lds_max = 65536;  // the device's LDS limit per workgroup
-  bool nt = true;          // streaming (non-temporal) accesses in the time-step kernels
-  bool force_terms = false;  // time-step kernels with the Guo terms also at F = 0
   int slab_planes = 0;       // AA steps in pairs as z-slabs of this many planes (0: whole box)
-  int odd_seg_w = 0;         // AA odd step as row segments of this width (k_dense_seg_odd; 0: off)
-  size_t odd_seg_lds = 0;    // its dynamic LDS floor (caps workgroups per CU)
-  int xk = 0;                // interleaved rows: nx / 64, split rows: nx / 2^xlg (0: plain rows)
-  int xlg = 6;
+  size_t odd_seg_lds = 0;    // dynamic LDS floor of the segmented odd step (caps workgroups per CU)
   int odd_ir_bx = 256;       // launch shape of the odd step on interleaved rows
   size_t odd_ir_lds = 0;
   lbm::PairKernel pair{};  // two time steps per launch (k_dense_pair); launch == nullptr: off
   lbm::PairArgs pair_args{};
-  bool walls = false;        // state through walls (K_AB_WALL), masked boxes in pairs
+  lbm::StepMode other;       // the mode the handle is not in
+  bool in_pairs = false;     // the present mode takes pairs
+  bool alone_ok = false;     // calls of one step may go back to the mode without pairs
+  bool starts_alone = false; // new states are written in the mode without pairs (restart)
+  int ones = 0, several = 0; // calls of one step in a row; steps of longer calls in a row
   bool own_capture = false;  // lbm_dense_graph_create is recording
   bool caller_graphs = false;  // a caller has recorded steps into a graph of its own
+  bool opp = true;           // AA: f_s(x) is in slot opp(s) at x (else gathered)
   int64_t ncell = 0, nfluid = 0, t = 0;
   size_t esize = 8;
   void* f[2] = {nullptr, nullptr};
