@@ -761,12 +761,51 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
   return p;
 }
 
+// Whether pairs of steps fill their tiles: rows of a tile past the box idle, and a
+// chunk collides two planes more than it finishes.  Measured (us per step, single /
+// pairs, 20 steps a call, boxes of 20,000 to 17M cells):
+//   FP64   ny = 2 111 / 118 (1024 x 2 x 1024), 3 167 / 132; nz = 1 214 / 234 (2048^2),
+//          2 17.4 / 19.2 (384^2), 3 650 / 548 (2048^2); D3Q27 ny = 2 as 3, nz = 3 938 /
+//          966, 4 on 3000 x 10 12.0 / 13.4, 6 122 / 97 (512^2), ny = 5 in tiles of 4 1,590
+//          / 1,670 (2048 x 5 x 2048), 6 471 / 372
+//   FP32   ny = 3 72.7 / 69.6 and D3Q27 113 / 119, 4 107 / 93 and 153 / 130; 9 rows in
+//          tiles of 8 54.4 / 59.2 and 75 / 91, 11 294 / 231 and 442 / 376; nz = 3 71.8 /
+//          75.0 (1024^2), 4 107 / 90
+//   FP16   gains little, so it needs nearly full tiles: 100^3 25.6 / 22.0, 96 x 100 x 90
+//          20.9 / 19.3; 17 rows 262 / 284 (1024 x 17 x 1024), 25 rows 342 / 358, 128 x
+//          128 x 16 8.7 / 10.0, 320 x 100 x 90 (lanes) 41.1 / 46.5; small boxes 48^3
+//          8.8 / 9.0, 64^3 10.2 / 9.2
+// Small boxes of a few planes are launch-bound and gain (256^2 x 1 FP64 8.5 / 5.2).
+//   masked AA, push: 128^2 x 24 FP64 22.6 / 20.1 and 21.4 / 20.1, x 12 12.8 / 12.6 and
+//          12.1 / 12.6, 100^2 x 20 14.0 / 14.4 and 12.4 / 14.4; large ones 512^2 x 8
+//          122 / 106, 6 72 / 81 (AA); the pull's single step is faster while both arrays
+//          fit the memory-side cache: 64^3 FP64 13.6 / 14.6, 80^3 25.9 / 28.0, 100^3
+//          69.1 / 57.5, D3Q27 FP32 channel 41.9 / 45.4, 128^3 87.8 / 69.9
+bool tiles_full(const lbm_dense* h, bool need_links) {
+  const int ty = h->q == 27 && h->storage == LBM_STORE_F64 ? 4 : 8;
+  const double rows = (double)h->ny / ((h->ny + ty - 1) / ty * ty);
+  if (h->storage == LBM_STORE_F16S) {
+    auto fill = [](int n, int w) { return (double)n / ((n + w - 1) / w * w); };
+    const int nc = h->nx / 2;
+    return h->ncell >= 250000 && rows * h->nz / (h->nz + 2.0) >= 0.9 &&
+           fill(nc, nc <= 32 ? 32 : 64) >= 0.85 * fill(h->nx, 64);
+  }
+  const bool f64 = h->storage == LBM_STORE_F64;
+  if (need_links)
+    return h->nz >= (h->ncell >= (1 << 21) ? 8 : 24) &&
+           (!h->pull || 2 * (size_t)h->ncell * h->q * h->esize > ((size_t)256 << 20));
+  if (h->ny < (f64 ? 3 : 4) || (h->ny > ty && rows < (f64 && h->q == 19 ? 0.0 : 0.65)))
+    return false;
+  if (h->ncell <= (1 << 17) && rows >= 0.9) return true;
+  return h->nz >= (!f64 ? 4 : (h->q == 19 ? 3 : 6));
+}
+
 // Two steps per launch (lbm_dense_pair.hpp) on SOA boxes in FP64, FP32 and (even
 // unmasked rows) FP16 deviations, without per-cell fields, and with a pressure drop only where there
 // is a mask.  Default from 20,000 cells on; below, the march along z is a longer chain than two
 // launches (us per step, one step / two steps per launch, D3Q19 FP64: 16^3 3.9 /
 // 4.6, 128 x 16 x 8 3.8 / 5.4, 24^3 5.0 / 4.8, 28^3 6.3 / 5.0, 12 x 12 x 200
-// 11.6 / 7.2; every larger size measured gained).  LBM_DENSE_PAIR=0|1 overrides;
+// 11.6 / 7.2), where they fill their tiles (tiles_full).  LBM_DENSE_PAIR=0|1 overrides;
 // a variable that tunes the one-step kernels asks for them.  Sets h->pair,
 // h->pair_args and the two-step mode, and the cache policy: stores stream past the caches when both
 // arrays exceed 320 MiB (100^3 FP64, 290 MiB: 44.0 us cached / 44.7 streaming;
@@ -786,6 +825,7 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
                         "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS", "LBM_DENSE_PUSH_GATHER",
                         "LBM_DENSE_FILL_SOLID"})
     on = on && !std::getenv(v);
+  on = on && tiles_full(h, need_links);
   if (e) on = e[0] != '0';
   const size_t plane_bytes = (size_t)h->nx * h->ny * h->esize;
   if (!on || h->layout != LBM_LAYOUT_SOA || cfg->tau || cfg->gamma ||
@@ -809,20 +849,13 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
   auto lanes = [](int columns, int w) { return (columns + w - 1) / w * w; };
   int v = 1;
   if (h->storage == LBM_STORE_F16S) {
-    // no kernel with one cell per lane; small boxes and tiles that would be half
-    // empty keep single steps (us per step, single / pairs: 64^3 D3Q19 10.2 / 9.2,
-    // 32^3 4.5 / 6.3, 100^3 D3Q27 33.2 / 29.7; 320 x 100 x 90 D3Q27, 17 % of the
-    // lanes empty, 58 / 65)
-    // The kernel works on scaled values: the scale has to be a power of two.
+    // No kernel with one cell per lane, and none for masks.  It works on scaled values:
+    // the scale has to be a power of two.
     v = 2;
-    const int nc = h->nx / 2;
     int exponent = 0;
     const double scale = cfg->f16_scale > 0.0 ? cfg->f16_scale : 4096.0;
     if (std::frexp(scale, &exponent) != 0.5 || std::abs(exponent) > 32) return;
-    if (h->nx % 2 || need_links ||
-        (!e && (h->ncell < (h->q == 19 ? 250000 : 500000) ||
-                nc < (h->q == 19 ? 0.75 : 0.85) * lanes(nc, nc <= 32 ? 32 : 64))))
-      return;
+    if (h->nx % 2 || need_links) return;
   } else if (h->storage == LBM_STORE_F32S && h->q == 19 && !need_links && h->nx % 2 == 0 &&
              h->ncell >= ((int64_t)1 << 22) && 2 * lanes(h->nx / 2, 64) <= lanes(h->nx, 64)) {
     v = 2;
