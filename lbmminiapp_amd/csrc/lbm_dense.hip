@@ -821,9 +821,12 @@ void choose_pair(lbm_dense* h, const lbm_dense_config* cfg, bool need_links, dou
                  StepMode* mode) {
   const char* e = std::getenv("LBM_DENSE_PAIR");
   bool on = h->ncell >= 20000;
-  for (const char* v : {"LBM_DENSE_IROWS", "LBM_DENSE_ODD_SEG", "LBM_DENSE_SLAB_PLANES",
-                        "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS", "LBM_DENSE_PUSH_GATHER",
-                        "LBM_DENSE_FILL_SOLID"})
+  for (const char* v : {"LBM_DENSE_IROWS", "LBM_DENSE_ODD_SEG", "LBM_DENSE_ODD_SEG_BLOCKS_PER_CU",
+                        "LBM_DENSE_SLAB_PLANES", "LBM_DENSE_STAGED", "LBM_DENSE_FORCE_TERMS",
+                        "LBM_DENSE_PUSH_GATHER", "LBM_DENSE_FILL_SOLID", "LBM_DENSE_BLOCK_X",
+                        "LBM_DENSE_BLOCKS_PER_CU", "LBM_DENSE_EVEN_BLOCK_X",
+                        "LBM_DENSE_EVEN_BLOCKS_PER_CU", "LBM_DENSE_ODD_IR_BLOCK_X",
+                        "LBM_DENSE_ODD_IR_BLOCKS_PER_CU"})
     on = on && !std::getenv(v);
   on = on && tiles_full(h, need_links);
   if (e) on = e[0] != '0';

@@ -1,5 +1,6 @@
-"""Two steps per launch asked for together with interleaved rows (LBM_DENSE_PAIR=1 and
-LBM_DENSE_IROWS=1): the states are those of single steps."""
+"""Switches that meet: two steps per launch asked for together with interleaved rows
+(LBM_DENSE_PAIR=1 and LBM_DENSE_IROWS=1) give the states of single steps; a variable that
+tunes the single-step kernels gives single steps."""
 import numpy as np
 import pytest
 
@@ -31,3 +32,16 @@ def test_pairs_with_interleaved_rows_asked_for(storage, masked, monkeypatch):
             out.append((lat.get_state(), *lat.moments(), lat.mass()))
     assert all(np.array_equal(a, b) for a, b in zip(out[0][:3], out[1][:3]))
     assert abs(out[0][3] - out[1][3]) <= 1e-12 * out[1][3]
+
+
+@pytest.mark.parametrize("name, value", [
+    ("BLOCK_X", "128"), ("BLOCKS_PER_CU", "4"), ("EVEN_BLOCK_X", "64"), ("EVEN_BLOCKS_PER_CU", "4"),
+    ("ODD_IR_BLOCK_X", "64"), ("ODD_IR_BLOCKS_PER_CU", "4"), ("ODD_SEG_BLOCKS_PER_CU", "4"), ("STAGED", "2")])
+def test_tuning_single_steps_asks_for_them(name, value, monkeypatch):
+    """An AA box of one array, as its device memory shows."""
+    one = 19 * 8 * 64 ** 3
+    with DenseLattice(64, 64, 64) as lat:
+        assert lat.info()["device_bytes"] > 2 * one
+    monkeypatch.setenv("LBM_DENSE_" + name, value)
+    with DenseLattice(64, 64, 64) as lat:
+        assert lat.info()["device_bytes"] < 2 * one
