@@ -952,7 +952,8 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   // Two steps per launch work out of place, in the AB pull convention.  For an AA
   // box they take a second population array, so only while both fit easily: a
   // quarter of the GPU's memory, and half of what is free (512^3 D3Q19 FP64:
-  // 41 of 288 GB).  Larger boxes, and a GPU that is nearly full, step in place.
+  // 41 of 288 GB), and a readback of the state, which takes q doubles per cell,
+  // beside them.  Larger boxes, and a GPU that is nearly full, step in place.
   StepMode paired;
   if (pair_ok) choose_pair(h, cfg, need_links, live, &paired);
   const size_t one_array = (size_t)h->ncell * h->q * h->esize;
@@ -960,7 +961,8 @@ lbm_status dense_create(const lbm_dense_config* cfg, lbm_dense** out, bool push_
   if (aa_as_pairs) {
     size_t room = 0, total = 0;
     if (hipMemGetInfo(&room, &total) != hipSuccess || 2 * one_array > total / 4 ||
-        2 * one_array > room / 2)
+        2 * one_array > room / 2 ||
+        2 * one_array + sizeof(double) * (size_t)h->ncell * h->q > room)
       h->pair = {};
   }
   // Interleaved rows (lbm_dense_kernels.hpp) for AA on unmasked periodic SOA
