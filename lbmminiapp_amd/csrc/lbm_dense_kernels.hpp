@@ -65,8 +65,8 @@ enum DenseKind {
 
 // Interleaved rows: position of x, x at position p, and the position of
 // x + d (d in {-1, 0, 1}, periodic) from the position p of x.  The same maps with
-// blocks of 2^lg positions and K = nx / 2^lg put x, x + K, x + 2K ... side by side
-// for the lanes of the two-step kernel that take several cells (split rows).
+// blocks of 2 positions (lg = 1) and K = nx / 2 put x and x + K side by side for the
+// lanes of the two-step kernel that take two cells (split rows).
 __host__ __device__ __forceinline__ int ir_pos(int x, int K, int lg = 6) {
   return ((x % K) << lg) + x / K;
 }
@@ -94,9 +94,16 @@ struct DenseArgs {
   double djump;                // density jump across the periodic x boundary (0: none)
   int z0;                      // first z-plane of the launch (z = blockIdx.z + z0): 0 except in
                                // the z-slab schedule of the AA steps
-  int xk;                      // interleaved rows: nx / 64 (split rows: nx / 2^xlg); 0: plain rows
-  int xlg;                     // log2 of the block (6, or split rows: 1, 2)
+  int xk;                      // interleaved rows: nx / 64 (split rows: nx / 2); 0: plain rows
+  int xlg;                     // log2 of the block (6, or split rows: 1)
 };
+
+// Whether masked boxes have a two-step kernel, and so states through walls: FP16 has
+// none, and in D3Q27 FP64 it spills in every tile shape.
+template <int Q, int STORE>
+constexpr bool masked_pairs() {
+  return STORE == LBM_STORE_F32S || (STORE == LBM_STORE_F64 && Q == 19);
+}
 
 // Pressure-drop boundary: the value a population carries across the periodic
 // x boundary changes by sign * w_s * djump (sign +1 forward, from x = nx - 1 to
@@ -910,7 +917,7 @@ DenseLaunchFn pick_kind(int kind, bool mask, bool force) {
     case K_AB_PUSH: return pick_flags<Q, STORE, LAYOUT, K_AB_PUSH, NT>(mask, force);
     case K_AB_PULL: return pick_flags<Q, STORE, LAYOUT, K_AB_PULL, NT>(mask, force);
     case K_AB_WALL:
-      if constexpr (LAYOUT == LBM_LAYOUT_SOA) {
+      if constexpr (LAYOUT == LBM_LAYOUT_SOA && masked_pairs<Q, STORE>()) {
         if (!mask) return nullptr;
         return force ? launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, true, NT>
                      : launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, false, NT>;

@@ -498,9 +498,10 @@ PairKernel pick_pair_flags(bool force, bool nt) {
 // tile and has no two-step kernel.
 template <int Q, int STORE, bool MASK, int V>
 PairKernel pick_pair_tile(bool force, bool nt, bool narrow, bool small) {
-  if constexpr (MASK && STORE == LBM_STORE_F64) {
-    if constexpr (Q == 27) return {};
-    else return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 10, V>(force, nt)
+  if constexpr (MASK && !masked_pairs<Q, STORE>()) {
+    return {};
+  } else if constexpr (MASK && STORE == LBM_STORE_F64) {
+    return narrow ? pick_pair_flags<Q, STORE, MASK, 32, 10, V>(force, nt)
                        : pick_pair_flags<Q, STORE, MASK, 64, 5, V>(force, nt);
   } else {
     if constexpr (!(Q == 27 && STORE == LBM_STORE_F64)) {
