@@ -31,16 +31,24 @@ def test_large_readback_equals_parts(size):
 
 
 def test_large_adjoint_states_f32():
-    size = (96, 90, 47)
+    """An FP32 adjoint state above the size that is staged from the first copy on (32 MiB of
+    floats), not a multiple of a chunk, piece or word, against the FP64 adjoint cell by cell: the
+    state is random, so a piece put in another place differs by as much as the values."""
+    size = (101, 97, 53)
     n = size[0] * size[1] * size[2]
-    gamma = np.zeros(n)
-    with Adjoint(*size, storage="f32s", gamma=gamma, checkpoint_every=2) as adj:
-        f = 0.05 + 0.01 * np.random.default_rng(5).random((19, n))
-        adj.set_initial_state(f)
-        print("[readback] adjoint f32s", flush=True)
-        adj.forward(2)
-        adj.backward()
-        lam = adj.lambda0()
-        small = adj.lambda0()
-        assert np.array_equal(lam, small) and np.array_equal(lam, lam.astype(np.float32))
-        assert np.isfinite(lam).all() and np.abs(lam).max() > 0
+    assert 19 * n * 4 > 32 << 20 and 19 * n * 4 % (1 << 20) and 19 * n * 4 % 16
+    f = 0.05 + 0.01 * np.random.default_rng(5).random((19, n))
+    lam = {}
+    for storage in ("f64", "f32s"):
+        with Adjoint(*size, storage=storage, gamma=np.zeros(n), checkpoint_every=2) as adj:
+            adj.set_initial_state(f)
+            print(f"[readback] adjoint {storage}", flush=True)
+            adj.forward(2)
+            adj.backward()
+            lam[storage] = adj.lambda0()
+            assert np.array_equal(adj.lambda0(), lam[storage])
+    big = np.abs(lam["f64"]).max()
+    assert np.array_equal(lam["f32s"], lam["f32s"].astype(np.float32))
+    # two steps of some tens of FP32 operations: a few tens of ulps of the largest value
+    assert np.abs(lam["f32s"] - lam["f64"]).max() <= 64 * 2.0 ** -24 * big
+    assert np.abs(np.diff(lam["f64"].reshape(-1))).mean() > 1e-2 * big
