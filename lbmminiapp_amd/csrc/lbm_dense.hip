@@ -624,7 +624,8 @@ lbm_status enqueue_step(lbm_dense* h) {
     st = launch_kind(h, h->opp ? K_AA_EVEN : K_AA_ODD, h->f[h->cur], h->f[h->cur]);
     h->opp = !h->opp;
   } else {
-    st = launch_kind(h, h->walls ? K_AB_WALL : (h->pull ? K_AB_PULL : K_AB_PUSH), h->f[h->cur],
+    const int pull = h->xk && h->xlg == 1 ? K_AB_PULL_SPLIT : K_AB_PULL;
+    st = launch_kind(h, h->walls ? K_AB_WALL : (h->pull ? pull : K_AB_PUSH), h->f[h->cur],
                      h->f[1 - h->cur]);
     h->cur = 1 - h->cur;
   }

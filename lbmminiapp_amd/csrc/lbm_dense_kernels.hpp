@@ -58,9 +58,10 @@ namespace lbm {
 
 constexpr uint32_t SOLID_BIT = 1u << 31;
 
-// K_AA_ODD_IR: the AA odd step on interleaved rows
+// K_AA_ODD_IR: the AA odd step on interleaved rows; K_AB_PULL_SPLIT: the pull on split rows
 enum DenseKind {
-  K_AA_EVEN = 0, K_AA_ODD = 1, K_AB_PUSH = 2, K_AB_PULL = 3, K_AA_ODD_IR = 4, K_AB_WALL = 5
+  K_AA_EVEN = 0, K_AA_ODD = 1, K_AB_PUSH = 2, K_AB_PULL = 3, K_AA_ODD_IR = 4, K_AB_WALL = 5,
+  K_AB_PULL_SPLIT = 6
 };
 
 // Interleaved rows: position of x, x at position p, and the position of
@@ -103,6 +104,12 @@ struct DenseArgs {
 template <int Q, int STORE>
 constexpr bool masked_pairs() {
   return STORE == LBM_STORE_F32S || (STORE == LBM_STORE_F64 && Q == 19);
+}
+
+// Whether the two-step kernels of unmasked boxes may take two cells per lane.
+template <int Q, int STORE>
+constexpr bool split_rows() {
+  return STORE == LBM_STORE_F16S || (STORE == LBM_STORE_F32S && Q == 19);
 }
 
 // Pressure-drop boundary: the value a population carries across the periodic
@@ -332,17 +339,20 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
     k_dense(const typename Storage<STORE>::T* f0, typename Storage<STORE>::T* f1, DenseArgs a) {
   using C = typename Storage<STORE>::C;
   constexpr bool IR = KIND == K_AA_ODD_IR;
-  constexpr bool WALL = KIND == K_AB_WALL;
-  static_assert(!IR || (!MASK && LAYOUT == LBM_LAYOUT_SOA), "interleaved rows: unmasked SOA only");
+  constexpr bool WALL = KIND == K_AB_WALL, SPLIT = KIND == K_AB_PULL_SPLIT;
+  static_assert(!(IR || SPLIT) || (!MASK && LAYOUT == LBM_LAYOUT_SOA),
+                "interleaved and split rows: unmasked SOA only");
   static_assert(!WALL || (MASK && LAYOUT == LBM_LAYOUT_SOA), "through-wall slots: masked SOA only");
   // x: the thread's row position (on interleaved rows, a.xk != 0, element xr
   // of the row).  Interleaved rows make every x-shifted access one aligned
   // block as well (see the file comment).
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= a.nx) return;
-  const int lg = IR ? 6 : a.xlg;
+  // log2 of the row block; known here, since this arithmetic starts every step of a
+  // small box (read from the arguments: 16 x 39 x 21 D3Q19 FP64 push 5.17 us, now 4.91)
+  constexpr int lg = SPLIT ? 1 : 6;
   const int xr = a.xk ? ir_x(x, a.xk, lg) : x;
-  const bool permuted = IR || a.xk != 0, irows = permuted && lg == 6;
+  const bool permuted = IR || SPLIT || a.xk != 0, irows = permuted && lg == 6;
   const int y = blockIdx.y, z = blockIdx.z + a.z0;
   const int64_t cell = x + (int64_t)a.nx * (y + (int64_t)a.ny * z);
   uint32_t lk = 0;
@@ -386,7 +396,7 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
           yy = wrap1(y - cy, a.ny);
           zz = wrap1(z - cz, a.nz);
           cross = gather_crossing(cx, xr, a.nx);
-        } else if constexpr (KIND == K_AA_ODD || KIND == K_AB_PULL) {
+        } else if constexpr (KIND == K_AA_ODD || KIND == K_AB_PULL || SPLIT) {
           aligned = cx == 0 || irows;
           xx = permuted ? ir_shift(x, -cx, a.xk, lg) : wrap1(x - cx, a.nx);
           yy = wrap1(y - cy, a.ny);
@@ -433,7 +443,7 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
     for (int s = 0; s < Q; s++) {
       const int o = Lattice<Q>::opp(s);
       const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
-      if constexpr (KIND == K_AA_EVEN || KIND == K_AB_PULL) {
+      if constexpr (KIND == K_AA_EVEN || KIND == K_AB_PULL || SPLIT) {
         put_row(row_of(f1, n, s, a, y, z), x, d[s], true);
       } else if constexpr (IR) {
         put_row(row_of(f1, n, o, a, wrap1(y + cy, a.ny), wrap1(z + cz, a.nz)), ir_shift(x, cx, a.xk),
@@ -455,7 +465,7 @@ __global__ void __launch_bounds__(kDenseMaxBlock)
   for (int s = 0; s < Q; s++) {
     const int o = Lattice<Q>::opp(s);
     const int cx = Lattice<Q>::c(s, 0), cy = Lattice<Q>::c(s, 1), cz = Lattice<Q>::c(s, 2);
-    if constexpr (KIND == K_AA_EVEN || KIND == K_AB_PULL) {
+    if constexpr (KIND == K_AA_EVEN || KIND == K_AB_PULL || SPLIT) {
       put(slot<Q, LAYOUT>(n, s, cell), solid ? C(0) : d[s], true);
     } else if constexpr (WALL) {
       // Slot s at x belongs to the cell beyond a blocked link where that cell is
@@ -921,6 +931,13 @@ DenseLaunchFn pick_kind(int kind, bool mask, bool force) {
         if (!mask) return nullptr;
         return force ? launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, true, NT>
                      : launch_dense<Q, STORE, LAYOUT, K_AB_WALL, true, false, NT>;
+      }
+      return nullptr;
+    case K_AB_PULL_SPLIT:
+      if constexpr (LAYOUT == LBM_LAYOUT_SOA && split_rows<Q, STORE>()) {
+        if (mask) return nullptr;
+        return force ? launch_dense<Q, STORE, LAYOUT, K_AB_PULL_SPLIT, false, true, NT>
+                     : launch_dense<Q, STORE, LAYOUT, K_AB_PULL_SPLIT, false, false, NT>;
       }
       return nullptr;
     case K_AA_ODD_IR:
