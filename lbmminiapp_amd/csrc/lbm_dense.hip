@@ -775,8 +775,11 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
 //   FP16   gains little, so it needs nearly full tiles: 100^3 25.6 / 22.0, 96 x 100 x 90
 //          20.9 / 19.3; 17 rows 262 / 284 (1024 x 17 x 1024), 25 rows 342 / 358, 128 x
 //          128 x 16 8.7 / 10.0, 320 x 100 x 90 (lanes) 41.1 / 46.5; small boxes 48^3
-//          8.8 / 9.0, 64^3 10.2 / 9.2
-// Small boxes of a few planes are launch-bound and gain (256^2 x 1 FP64 8.5 / 5.2).
+//          8.8 / 9.0, 64^3 10.2 / 9.2; AB 64^3 7.5 / 9.3, 128^3 27.4 / 27.6, 256 x 200 x
+//          128 93.3 / 79.2
+// Small boxes of a few planes are launch-bound and gain (256^2 x 1 FP64 8.5 / 5.2), but the
+// smallest ones wait for the march along z (64 x 64 x 12 FP32 4.4 / 4.7, 79 x 14 x 47 pull
+// FP64 with a force 8.2 / 9.6, 28^3 5.9 / 5.5).
 //   masked AA, push: 128^2 x 24 FP64 22.6 / 20.1 and 21.4 / 20.1, x 12 12.8 / 12.6 and
 //          12.1 / 12.6, 100^2 x 20 14.0 / 14.4 and 12.4 / 14.4; large ones 512^2 x 8
 //          122 / 106, 6 72 / 81 (AA); the pull's single step is faster while both arrays
@@ -785,16 +788,18 @@ PairArgs plan_pair(const PairKernel& k, int nx, int ny, int nz, int slots) {
 bool tiles_full(const lbm_dense* h, bool need_links) {
   const int ty = h->q == 27 && h->storage == LBM_STORE_F64 ? 4 : 8;
   const double rows = (double)h->ny / ((h->ny + ty - 1) / ty * ty);
+  const bool ab = h->pattern == LBM_PATTERN_AB;
+  const bool past_cache = 2 * (size_t)h->ncell * h->q * h->esize > ((size_t)256 << 20);
   if (h->storage == LBM_STORE_F16S) {
     auto fill = [](int n, int w) { return (double)n / ((n + w - 1) / w * w); };
     const int nc = h->nx / 2;
-    return h->ncell >= 250000 && rows * h->nz / (h->nz + 2.0) >= 0.9 &&
+    return (ab ? past_cache : h->ncell >= 250000) && rows * h->nz / (h->nz + 2.0) >= 0.9 &&
            fill(nc, nc <= 32 ? 32 : 64) >= 0.85 * fill(h->nx, 64);
   }
   const bool f64 = h->storage == LBM_STORE_F64;
   if (need_links)
-    return h->nz >= (h->ncell >= (1 << 21) ? 8 : 24) &&
-           (!h->pull || 2 * (size_t)h->ncell * h->q * h->esize > ((size_t)256 << 20));
+    return h->nz >= (h->ncell >= (1 << 21) ? 8 : 24) && (!h->pull || past_cache);
+  if (h->ncell < 60000 && (rows < 0.9 || h->nz < 16)) return false;
   if (h->ny < (f64 ? 3 : 4) || (h->ny > ty && rows < (f64 && h->q == 19 ? 0.0 : 0.65)))
     return false;
   if (h->ncell <= (1 << 17) && rows >= 0.9) return true;

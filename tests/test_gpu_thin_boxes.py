@@ -16,6 +16,7 @@ CASES = [  # size, storage, D3Q, pairs
     ((512, 512, 3), "f32s", 19, False), ((512, 512, 4), "f32s", 19, True), ((256, 256, 1), "f64", 19, True),
     ((100000, 1, 1), "f32s", 27, False), ((128, 128, 16), "f16s", 19, False), ((320, 100, 90), "f16s", 27, False),
     ((120, 17, 300), "f16s", 19, False), ((80, 80, 80), "f16s", 27, True),
+    ((64, 64, 12), "f32s", 19, False), ((79, 14, 47), "f64", 19, False), ((32, 32, 32), "f32s", 27, True),
 ]
 
 
