@@ -200,7 +200,9 @@ lbm_status lbm_dense_init_tgv(lbm_dense* h, double u0, double noise, uint64_t se
  * A handle that can take two steps per launch does so for calls of two and more; calls
  * of one step in a row go back to single steps in the way of its pattern (AA: in place)
  * where that is the faster one, at the third of them, and calls of more steps back into
- * pairs, once 8 steps have been asked for.  A change costs about a step and a half. */
+ * pairs, once 8 steps have been asked for.  A change costs one and a half to three
+ * steps.  Steps that a caller captures into a graph of its own fix the way from then
+ * on (lbm_dense_set_stream). */
 lbm_status lbm_dense_step(lbm_dense* h, int32_t nsteps);
 /* Advance n steps and return their device time (HIP events on the handle's stream). */
 lbm_status lbm_dense_run_timed(lbm_dense* h, int32_t nsteps, double* elapsed_ms);
@@ -219,7 +221,10 @@ lbm_status lbm_dense_synchronize(lbm_dense* h);
  * lbm_dense_set_stream: enqueue every later call on `stream` (a hipStream_t;
  * NULL returns to the handle's own stream).  Waits for the work already
  * enqueued on the previous stream.  The stream must outlive its use by the
- * handle.
+ * handle.  Steps captured from it into a caller's own graph replay on the arrays
+ * they were captured with: whatever is called between replays, an even run then
+ * ends in the array it started in (for that it takes two steps per launch four
+ * steps at a time), and the way of stepping stays the one at capture.
  *
  * lbm_dense_graph_create: capture `nsteps` time steps (even, > 0) as a HIP graph
  * of kernel launches only (no memory-set or copy nodes).  Nothing runs and the

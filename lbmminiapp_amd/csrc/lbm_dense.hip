@@ -232,11 +232,14 @@ __global__ void __launch_bounds__(256)
 }
 
 // The state of every fluid cell from one gathering convention and row order into
-// another, in another array; values as they are stored.
+// another, in another array; values as they are stored.  Bound by the accesses of the
+// side whose rows are permuted (512^3, plain or split to interleaved rows: FP64 10.2
+// ms, FP32 6.6, FP16 5.8).
 template <int Q, int STORE, int LAYOUT>
 __global__ void __launch_bounds__(256)
     k_convert(const void* __restrict__ src, DenseArgs sa, int smode, void* __restrict__ dst,
               DenseArgs da, int dmode) {
+  if constexpr (LAYOUT != LBM_LAYOUT_SOA) return;
   using T = typename Storage<STORE>::T;
   int x, y, z;
   int64_t cell;
@@ -244,9 +247,25 @@ __global__ void __launch_bounds__(256)
   const uint32_t lk = sa.links ? sa.links[cell] : 0u;  // (masked boxes: plain rows)
   if (lk & SOLID_BIT) return;
   const Offsets off(x, y, z, sa.nx, sa.ny, sa.nz);
-  for (int s = 0; s < Q; s++)
-    static_cast<T*>(dst)[canon_index<Q, LAYOUT>(dmode, s, cell, x, lk, off, da)] =
-        static_cast<const T*>(src)[canon_index<Q, LAYOUT>(smode, s, cell, x, lk, off, sa)];
+  // positions of x - 1, x and x + 1 in the rows of both sides
+  int from[3], to[3];
+  for (int i = 0; i < 3; i++) {
+    const int xx = wrap1(x + i - 1, sa.nx);
+    from[i] = sa.xk ? ir_pos(xx, sa.xk, sa.xlg) : xx;
+    to[i] = da.xk ? ir_pos(xx, da.xk, da.xlg) : xx;
+  }
+  const int64_t n = sa.ncell, row = cell - x;
+#pragma unroll
+  for (int s = 0; s < Q; s++) {
+    const int o = Lattice<Q>::opp(s), cx = Lattice<Q>::c(s, 0);
+    const int64_t there = slot<Q, LAYOUT>(
+        n, s, row + off.oy[1 - Lattice<Q>::c(s, 1)] + off.oz[1 - Lattice<Q>::c(s, 2)]);
+    const int64_t back = slot<Q, LAYOUT>(n, o, row);
+    const bool blocked = (lk >> o) & 1u;
+    const int64_t i = blocked && smode == C_GATHER ? back + from[1] : there + from[1 - cx];
+    const int64_t j = blocked && dmode == C_GATHER ? back + to[1] : there + to[1 - cx];
+    static_cast<T*>(dst)[j] = static_cast<const T*>(src)[i];
+  }
 }
 
 // ---------------------------------------------------------------- mass
@@ -635,9 +654,9 @@ lbm_status enqueue_step(lbm_dense* h) {
 
 // The mode for a call of `nsteps` steps; takes the first of them where the state has
 // to leave the AA even convention (whose stored values include the pressure jump)
-// before it can go into pairs.  A change of mode costs about a step and a half, so a
-// handle changes when the calls of a kind repeat: to pairs for 8 steps asked for in
-// calls of two and more, back at the third call of one step in a row.
+// before it can go into pairs.  A change of mode costs one and a half (FP64) to three
+// (FP16) steps, so a handle changes when the calls of a kind repeat: to pairs for 8
+// steps asked for in calls of two and more, back at the third call of one step in a row.
 lbm_status choose_mode(lbm_dense* h, int nsteps, int* taken) {
   h->ones = nsteps == 1 ? h->ones + 1 : 0;
   h->several = nsteps == 1 ? 0 : std::min(h->several + nsteps, 8);
