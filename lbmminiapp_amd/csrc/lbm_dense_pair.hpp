@@ -10,7 +10,8 @@
 // s at x - c_s), out of place: reads are the x-shifted ones and go through the
 // caches, where neighbouring workgroups share them; writes are whole aligned
 // row segments.  A handle that the caller created as AA or AB push runs it too
-// (dense_create): every convention holds the same states, bit for bit.
+// (dense_create): every convention holds the same states, bit for bit (k_convert
+// moves them).
 //
 // A workgroup owns a tile of W x TY cells in (x, y) and marches along z through
 // a chunk of lz planes.  At plane p it
@@ -23,9 +24,9 @@
 //      c_z = 0 and c_z > 0 parts wait in registers for planes p and p + 1.
 // One plane of the Q - 3 exchanged directions is all the LDS holds, so the tile
 // can be large: the ring costs (W + 2)(TY + 2) / (W TY), 1.29 for 64 x 8, in
-// the first step's arithmetic; in memory traffic the caches absorb most of it
-// (measured, 512^3 D3Q19 FP64: 23.0 GB read where the state is 20.4, 20.4
-// written).
+// the first step's arithmetic; in memory traffic the caches absorb part of it
+// (measured, 512^3 D3Q19 FP64: 24 to 26 GB read per launch where the state is 20.4,
+// 20.4 written).
 //
 // Waves: W TY / 64 of tile rows, 2 W / 64 of the rows above and below, one of
 // the two columns beside the tile.  Only the tile's waves do the second step.
@@ -57,7 +58,7 @@
 // 968 us per step; now 628, single steps 763).
 //
 // Measured, ms per step, one-step kernels -> pairs (tile as choose_pair takes it):
-//   D3Q19 FP64 512^3 7.15 -> 4.10   256^3 0.912 -> 0.493   128^3 0.110 -> 0.067
+//   D3Q19 FP64 512^3 7.08 -> 4.00 to 4.23   256^3 0.970 -> 0.493   128^3 0.110 -> 0.069
 //   D3Q19 FP32 512^3 3.39 -> 2.05   256^3 0.424 -> 0.268
 //   D3Q19 FP16 512^3 1.74 -> 1.45   256^3 0.219 -> 0.186   D3Q27 FP16 256^3 0.325 -> 0.263
 //   D3Q27 FP64 384^3 4.44 -> 3.09   FP32 256^3 0.635 -> 0.414
