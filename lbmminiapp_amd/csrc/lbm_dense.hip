@@ -235,11 +235,10 @@ __global__ void __launch_bounds__(256)
 // another, in another array; values as they are stored.  Bound by the accesses of the
 // side whose rows are permuted (512^3, plain or split to interleaved rows: FP64 10.2
 // ms, FP32 6.6, FP16 5.8).
-template <int Q, int STORE, int LAYOUT>
+template <int Q, int STORE>
 __global__ void __launch_bounds__(256)
     k_convert(const void* __restrict__ src, DenseArgs sa, int smode, void* __restrict__ dst,
               DenseArgs da, int dmode) {
-  if constexpr (LAYOUT != LBM_LAYOUT_SOA) return;
   using T = typename Storage<STORE>::T;
   int x, y, z;
   int64_t cell;
@@ -258,9 +257,9 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int s = 0; s < Q; s++) {
     const int o = Lattice<Q>::opp(s), cx = Lattice<Q>::c(s, 0);
-    const int64_t there = slot<Q, LAYOUT>(
+    const int64_t there = slot<Q, LBM_LAYOUT_SOA>(
         n, s, row + off.oy[1 - Lattice<Q>::c(s, 1)] + off.oz[1 - Lattice<Q>::c(s, 2)]);
-    const int64_t back = slot<Q, LAYOUT>(n, o, row);
+    const int64_t back = slot<Q, LBM_LAYOUT_SOA>(n, o, row);
     const bool blocked = (lk >> o) & 1u;
     const int64_t i = blocked && smode == C_GATHER ? back + from[1] : there + from[1 - cx];
     const int64_t j = blocked && dmode == C_GATHER ? back + to[1] : there + to[1 - cx];
@@ -348,8 +347,14 @@ LBM_UTIL_KERNEL(k_get_canonical)
 LBM_UTIL_KERNEL(k_moments)
 LBM_UTIL_KERNEL(k_init)
 LBM_UTIL_KERNEL(k_mass_partial)
-LBM_UTIL_KERNEL(k_convert)
 #undef LBM_UTIL_KERNEL
+template <int Q, int S, int L>
+struct k_convert_u {  // SOA boxes only: the ones that have two-step launches
+  template <typename... A>
+  static void launch(dim3 g, dim3 b, hipStream_t st, A... a) {
+    if constexpr (L == LBM_LAYOUT_SOA) hipLaunchKernelGGL((k_convert<Q, S>), g, b, 0, st, a...);
+  }
+};
 
 }  // namespace lbm
 

@@ -45,3 +45,19 @@ def test_tuning_single_steps_asks_for_them(name, value, monkeypatch):
     monkeypatch.setenv("LBM_DENSE_" + name, value)
     with DenseLattice(64, 64, 64) as lat:
         assert lat.info()["device_bytes"] < 2 * one
+
+
+@pytest.mark.parametrize("scale, pairs", [(1000.0, False), (4096.0, True), (1024.0, True)])
+def test_fp16_pairs_need_a_power_of_two(scale, pairs, monkeypatch):
+    """The two-step kernel works on scaled values; another scale takes single steps (one array)."""
+    size, out = (66, 10, 9), []
+    one = 19 * 2 * size[0] * size[1] * size[2]
+    for pair in "10":
+        monkeypatch.setenv("LBM_DENSE_PAIR", pair)
+        print(f"[switches] f16 scale {scale} pair={pair}", flush=True)
+        with DenseLattice(*size, storage="f16s", f16_scale=scale, omega=1 / 0.8) as lat:
+            assert (lat.info()["device_bytes"] > 2 * one) == (pairs and pair == "1")
+            lat.init_tgv(0.05, 1e-3, 3)
+            lat.step(5)
+            out.append((lat.get_state(), *lat.moments()))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
