@@ -9,8 +9,8 @@ Compiler flags:
   --offload-arch=gfx950                  MI355X only, no other targets
   -ffp-contract=off                      no implicit FMA: the FP64 path must be the
                                          reference's IEEE operation sequence; the
-                                         reduced-precision collision re-enables
-                                         contraction locally with a pragma
+                                         reduced-precision collision writes its
+                                         FMAs out
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                          no packed FP32 instructions
 """
